@@ -37,13 +37,24 @@ __global__ __launch_bounds__(256) void k_gather(
 }
 
 // CSR cell ranges straight from the sorted keys, no scan: the key in slot s starts its run when
-// the key before it, pk, differs; slot s then writes cell_start[c] = s for the cells
+// the key before it, pk, differs; slot s then owns cell_start[c] = s for the cells
 // pk < c <= k (the empty cells before its own take its index: the first sorted index with key
-// >= c), and the last slot also writes n for the cells after its key up to and including C.
-// These ranges partition 0..C, so every entry is written once; together they are the prefix
-// sum of the per-cell counts of hashgrid.rs:102-106.  Short ranges are written by their lane,
-// long ones by the whole wave.
-__device__ __forceinline__ void fill_cells(uint32_t* __restrict__ cell_start, uint32_t lo,
+// >= c), and the last slot also owns the cells after its key up to and including C, which take
+// n.  These ranges partition 0..C, so every entry is written once; together they are the prefix
+// sum of the per-cell counts of hashgrid.rs:102-106.
+//
+// A slot's wave writes its ranges except the blocks of kCellBlock cells (aligned, the last one
+// ending at C) that lie wholly inside one range: those are empty cells between two runs, and the
+// lanes of fill_empty_blocks write them.  Left to the slot, a long gap is one wave's
+// serial store loop: a dam-break block of 1,048,576 particles in the lower part of 100^3 cells
+// leaves ~680,000 cells behind its last key, and k_gather_resident took 312 us with them against
+// 14 us now (k_cell_starts 304 -> 6 us).  What a slot keeps of a gap
+// is at most two partial blocks.
+constexpr uint32_t kCellBlock = 256;
+
+// cell_start[lo..hi) = val without the whole blocks inside (C1 = C + 1 entries in all).  Short
+// ranges are written by their lane, longer ones by the whole wave.
+__device__ __forceinline__ void fill_range(uint32_t* __restrict__ cell_start, uint32_t lo,
                                            uint32_t hi, uint32_t val, int lane) {
     const bool mine = hi - lo <= 8u;
     if (mine)
@@ -58,6 +69,44 @@ __device__ __forceinline__ void fill_cells(uint32_t* __restrict__ cell_start, ui
         for (uint32_t c = wlo + (uint32_t)lane; c < whi; c += kWave) cell_start[c] = wv;
     }
 }
+__device__ __forceinline__ void fill_cells(uint32_t* __restrict__ cell_start, uint32_t lo,
+                                           uint32_t hi, uint32_t C1, uint32_t val, int lane) {
+    const uint32_t first = (lo + kCellBlock - 1u) & ~(kCellBlock - 1u);  // may wrap past 2^32
+    const uint32_t end = hi == C1 ? hi : hi & ~(kCellBlock - 1u);
+    const bool cut = first >= lo && first < end;  // whole blocks [first, end) are not ours
+    fill_range(cell_start, lo, cut ? first : hi, val, lane);
+    if (__ballot(cut && end < hi) != 0ull)
+        fill_range(cell_start, cut ? end : hi, hi, val, lane);
+}
+
+// Blocks of kCellBlock cells, 16 lanes each: a block is written when no key falls in it before
+// its last cell, i.e. when it lies inside one slot's range (the rule fill_cells skips by).  The
+// first slot whose key is >= the block's first cell is searched with 16 probes per round: six
+// dependent rounds for 4,194,304 keys, a third of the loads that 64 probes take in four.  These
+// workgroups come first in the launch, so that the rounds overlap the slots' work (a grid with no
+// long gap pays 0.8 us: 551,368 cells of 4,194,304 uniform points, k_csr_from_sorted 8.7 -> 9.5).
+constexpr uint32_t kBlockLanes = 16, kGroupBlocks16 = 256 / kBlockLanes;
+__device__ __forceinline__ void fill_empty_blocks(uint32_t group, const uint32_t* __restrict__ keys,
+                                                  uint32_t n, uint32_t C,
+                                                  uint32_t* __restrict__ cell_start) {
+    const uint32_t b = group * kGroupBlocks16 + threadIdx.x / kBlockLanes;
+    const uint32_t t = threadIdx.x % kBlockLanes, shift = (threadIdx.x & 63u) & ~(kBlockLanes - 1u);
+    const bool live = b <= C / kCellBlock;
+    const uint32_t c0 = live ? b * kCellBlock : 0u, last = min(c0 + (kCellBlock - 1u), C);
+    uint32_t lo = 0, hi = live ? n : 0u;
+    while (__ballot(lo < hi) != 0ull) {  // until every block of the wave has its slot
+        const uint32_t step = (hi - lo + kBlockLanes - 1u) / kBlockLanes;
+        const uint32_t i = lo + t * step;
+        const bool less = i < hi && keys[min(i, n - 1u)] < c0;
+        const uint32_t below =
+            (uint32_t)__popcll((__ballot(less) >> shift) & ((1ull << kBlockLanes) - 1ull));
+        hi = below ? min(hi, lo + below * step) : lo;
+        lo += below ? (below - 1u) * step + 1u : 0u;
+    }
+    if (!live || (lo < n && keys[lo] < last)) return;
+    for (uint32_t c = t; c <= last - c0; c += kBlockLanes) cell_start[c0 + c] = lo;
+}
+static uint32_t empty_block_groups(uint32_t C) { return C / (kGroupBlocks16 * kCellBlock) + 1u; }
 
 // Cell ranges, and (big != null) the candidate co-located groups: runs of at least
 // kCollapseMin keys in which at least kGroupHits of kGroupSamples evenly spaced particles (over
@@ -88,8 +137,8 @@ __device__ __forceinline__ void cell_starts_slot(uint32_t s, const uint32_t* __r
             hi2 = C + 1u;
         }
     }
-    fill_cells(cell_start, lo, hi, s, lane);
-    fill_cells(cell_start, lo2, hi2, n, lane);
+    fill_cells(cell_start, lo, hi, C + 1u, s, lane);
+    if (__ballot(lo2 < hi2) != 0ull) fill_cells(cell_start, lo2, hi2, C + 1u, n, lane);
     // Rare: a run of at least kCollapseMin.  The whole wave takes each such run of its lanes in
     // turn: lane q < kGroupSamples loads sample q (one round trip for all 16); the middle sample
     // is tried first as the group's position, then each other in turn (a corner group can fill
@@ -150,16 +199,21 @@ __global__ __launch_bounds__(256) void k_cell_starts(const uint32_t* __restrict_
                                                      const float4* __restrict__ spos,
                                                      uint2* __restrict__ big, uint32_t cap,
                                                      uint64_t* __restrict__ cand_tag,
-                                                     Control* ctl) {
-    cell_starts_slot(blockIdx.x * blockDim.x + threadIdx.x, skeys, n, C, cell_start,
+                                                     Control* ctl, uint32_t fill_groups) {
+    if (blockIdx.x < fill_groups) {
+        fill_empty_blocks(blockIdx.x, skeys, n, C, cell_start);
+        return;
+    }
+    cell_starts_slot((blockIdx.x - fill_groups) * blockDim.x + threadIdx.x, skeys, n, C, cell_start,
                      SortedPos{spos}, big, cap, cand_tag, ctl);
 }
 
 static hipError_t launch_cell_starts(fh_ctx* c, uint32_t cells, uint32_t n, bool list_big) {
+    const uint32_t fill = empty_block_groups(cells);
     tbeg(c, KID_SCAN);
-    k_cell_starts<<<ceil_div(n, 256u), 256, 0, c->stream>>>(
+    k_cell_starts<<<fill + ceil_div(n, 256u), 256, 0, c->stream>>>(
         c->skeys, n, cells, c->cell_start, c->spos, list_big ? c->big : nullptr,
-        ceil_div(c->max_n, 64u) + 1u, c->run_tag, c->ctl);
+        ceil_div(c->max_n, 64u) + 1u, c->run_tag, c->ctl, fill);
     tend(c, KID_SCAN);
     return hipGetLastError();
 }
@@ -185,8 +239,12 @@ __global__ __launch_bounds__(256) void k_gather_resident(
     const float4* __restrict__ sout, const uint32_t* __restrict__ prev, uint32_t n,
     float4* __restrict__ spos, float4* __restrict__ svel, const uint32_t* __restrict__ skeys,
     uint32_t C, uint32_t* __restrict__ cell_start, uint2* __restrict__ big, uint32_t cap,
-    uint64_t* __restrict__ cand_tag, Control* ctl) {
-    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+    uint64_t* __restrict__ cand_tag, Control* ctl, uint32_t fill_groups) {
+    if (blockIdx.x < fill_groups) {
+        fill_empty_blocks(blockIdx.x, skeys, n, C, cell_start);
+        return;
+    }
+    const uint32_t r = (blockIdx.x - fill_groups) * blockDim.x + threadIdx.x;
     if (r < n) {
         const uint32_t q = prev[r];
         if (q < n) {  // always, when the sort is consistent
@@ -201,10 +259,11 @@ __global__ __launch_bounds__(256) void k_gather_resident(
 
 hipError_t launch_gather_resident(fh_ctx* c, uint32_t cells, uint32_t n) {
     if (n == 0) return launch_fill_u32(c, c->cell_start, 0u, cells + 1u);
+    const uint32_t fill = empty_block_groups(cells);
     tbeg(c, KID_GATHER);
-    k_gather_resident<<<ceil_div(n, 256u), 256, 0, c->stream>>>(
+    k_gather_resident<<<fill + ceil_div(n, 256u), 256, 0, c->stream>>>(
         c->sout, c->sidx2, n, c->spos, c->svel, c->skeys, cells, c->cell_start, c->big,
-        ceil_div(c->max_n, 64u) + 1u, c->run_tag, c->ctl);
+        ceil_div(c->max_n, 64u) + 1u, c->run_tag, c->ctl, fill);
     tend(c, KID_GATHER);
     return hipGetLastError();
 }
@@ -213,11 +272,16 @@ hipError_t launch_gather_resident(fh_ctx* c, uint32_t cells, uint32_t n) {
 // array as the prefix sum of per-cell counts): cell_start[c] = number of keys < c for
 // c = 0..C, so keys >= C count in no cell.  Each slot fills the cells between the previous
 // slot's key and its own (both clamped to C), the last slot the cells after its key; the
-// filled ranges partition 0..C.
+// filled ranges partition 0..C (whole empty blocks: fill_empty_blocks).
 __global__ __launch_bounds__(256) void k_csr_from_sorted(const uint32_t* __restrict__ keys,
                                                          uint32_t n, uint32_t C,
-                                                         uint32_t* __restrict__ cell_start) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+                                                         uint32_t* __restrict__ cell_start,
+                                                         uint32_t fill_groups) {
+    if (blockIdx.x < fill_groups) {
+        fill_empty_blocks(blockIdx.x, keys, n, C, cell_start);
+        return;
+    }
+    const uint32_t s = (blockIdx.x - fill_groups) * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
     uint32_t lo = 0, hi = 0, lo2 = 0, hi2 = 0;
     if (s < n) {
@@ -230,14 +294,16 @@ __global__ __launch_bounds__(256) void k_csr_from_sorted(const uint32_t* __restr
             hi2 = C + 1u;
         }
     }
-    fill_cells(cell_start, lo, hi, s, lane);
-    fill_cells(cell_start, lo2, hi2, n, lane);
+    fill_cells(cell_start, lo, hi, C + 1u, s, lane);
+    if (__ballot(lo2 < hi2) != 0ull) fill_cells(cell_start, lo2, hi2, C + 1u, n, lane);
 }
 
 hipError_t launch_csr_from_sorted(fh_ctx* c, const uint32_t* keys, uint32_t n, uint32_t cells,
                                   uint32_t* cell_start) {
     if (n == 0) return launch_fill_u32(c, cell_start, 0u, cells + 1u);
-    k_csr_from_sorted<<<ceil_div(n, 256u), 256, 0, c->stream>>>(keys, n, cells, cell_start);
+    const uint32_t fill = empty_block_groups(cells);
+    k_csr_from_sorted<<<fill + ceil_div(n, 256u), 256, 0, c->stream>>>(
+        keys, n, cells, cell_start, fill);
     return hipGetLastError();
 }
 

@@ -76,6 +76,20 @@ def test_cell_start_csr_from_sorted_keys(fh, gpu_ctx, oracle, n, C):
         assert got[0].item() == 0 and fh.to_u32(got)[-1] == np.count_nonzero(keys < C)
 
 
+@pytest.mark.parametrize("C", [1, 255, 256, 257, 511, 1024, 100_000])
+@pytest.mark.parametrize("runs", [1, 2, 7, 300])
+def test_cell_start_csr_long_gaps(fh, gpu_ctx, oracle, C, runs):
+    """Runs of equal keys with long empty stretches before, between and behind them, their keys
+    at and beside the edges of the 256-cell blocks that are filled apart from the slots."""
+    rng = np.random.default_rng(1000 * runs + C)
+    edges = np.array([0, 1, 254, 255, 256, 257, 511, 512, 767, 768, C - 1, C, C + 5])
+    picks = np.concatenate([rng.choice(edges, (runs + 1) // 2), rng.integers(0, C + 2, runs // 2)])
+    keys = np.sort(np.repeat(np.maximum(picks, 0), rng.integers(1, 200, runs))).astype(np.uint32)
+    out = torch.full((C + 1,), -7, dtype=torch.int32, device="cuda")
+    got = fh.cell_start_csr(dev(keys.view(np.int32)), keys.size, C, out, ctx=gpu_ctx)
+    assert np.array_equal(fh.to_u32(got), oracle.cell_start_csr(keys, C))
+
+
 def pack_reference(frame, x, y, z):
     """serve.rs:43-62 FrameBuffer::set_frame on the interleaved positions of
     manifest_runner.rs:150-159: u32 LE frame, u32 LE count, f32 LE x0 y0 z0 x1 ..."""
