@@ -217,10 +217,12 @@ int fh_create(int device, uint32_t max_n, uint32_t max_cells, void* stream, fh_c
     c->max_sort_tiles = ceil_div(max_n, (uint32_t)kSortTile);
     size_t tot = 0;
     hipError_t e = hipSuccess;
-    if (e == hipSuccess) e = alloc(&c->ka, max_n, &tot);
-    if (e == hipSuccess) e = alloc(&c->va, max_n, &tot);
+    if (e == hipSuccess) e = alloc(&c->ka, 3 * (size_t)max_n, &tot);
+    if (e == hipSuccess) {
+        c->va = c->ka + max_n;
+        c->vb = c->ka + 2 * (size_t)max_n;
+    }
     if (e == hipSuccess) e = alloc(&c->kb, max_n, &tot);
-    if (e == hipSuccess) e = alloc(&c->vb, max_n, &tot);
     if (e == hipSuccess) e = alloc(&c->sort_lb, (size_t)c->max_sort_tiles * kDigitSlots, &tot);
     // a histogram row per kHistChunk keys, at most kHistBlocks rows (the histogram kernels'
     // grid for a sort of n <= max_n keys)
@@ -260,6 +262,7 @@ int fh_create(int device, uint32_t max_n, uint32_t max_cells, void* stream, fh_c
     if (e == hipSuccess)
         e = alloc(&c->lstream, 3 * (size_t)ceil_div(max_n, 64u) * kLightCacheWords, &tot);
     if (e == hipSuccess) e = alloc(&c->lstream_t, 3 * (size_t)ceil_div(max_n, 64u), &tot);
+    if (e == hipSuccess) e = alloc(&c->hits, 3 * (size_t)max_n, &tot);
     if (e == hipSuccess) e = alloc(&c->cell_grp, max_cells, &tot);
     if (e == hipSuccess) e = alloc(&c->big, (size_t)ceil_div(max_n, 64u) + 1u, &tot);
     if (e == hipSuccess) e = alloc(&c->skip_tag, (size_t)ceil_div(max_n, 64u), &tot);
@@ -316,9 +319,9 @@ int fh_destroy(fh_ctx* c) {
             delete[] t.ev;
         }
     }
-    void* bufs[] = {c->ka, c->va, c->kb, c->vb, c->sort_lb, c->ctl, c->run_tag,
+    void* bufs[] = {c->ka, c->kb, c->sort_lb, c->ctl, c->run_tag,
                     c->cell_start, c->skeys, c->sidx, c->spos, c->svel,
-                    c->srho, c->dpart, c->fpart, c->heavy, c->heavy_flag, c->hpart, c->hslot, c->lstream, c->lstream_t, c->hist_part,
+                    c->srho, c->dpart, c->fpart, c->heavy, c->heavy_flag, c->hpart, c->hslot, c->lstream, c->lstream_t, c->hits, c->hist_part,
                     c->sort_pre,
                     c->cell_grp, c->big, c->skip_tag, c->vrep, c->rank, c->sout,
                     c->sidx2};
@@ -500,7 +503,7 @@ int fh_sph_density(fh_ctx* c, const fh_sph_params* prm, const float* px, const f
         FH_CHECK_HIP(launch_density(c, a, c->cell_start, density));
     } else {
         FH_CHECK_HIP(launch_group_plan(c, a, false));
-        FH_CHECK_HIP(launch_density_fast(c, a, c->cell_start));
+        FH_CHECK_HIP(launch_density_fast(c, a, c->cell_start, false));
         FH_CHECK_HIP(launch_finalize(c, a, nullptr, true, nullptr, nullptr, nullptr, nullptr,
                                      nullptr, nullptr, density, nullptr));
     }
@@ -545,7 +548,7 @@ static int sph_fused_steps(fh_ctx* c, const fh_sph_params* prm, const fh_epilogu
         FH_CHECK_HIP(launch_group_plan(c, a, true));
         // pass timers: wall time of each pass (the force pass with its k_prep)
         tbeg(c, KID_DPASS);
-        FH_CHECK_HIP(launch_density_fast(c, a, c->cell_start));
+        FH_CHECK_HIP(launch_density_fast(c, a, c->cell_start, true));
         tend(c, KID_DPASS);
         tbeg(c, KID_FPASS);
         FH_CHECK_HIP(launch_prep(c, a));

@@ -99,6 +99,10 @@ constexpr int kHeavyComps = 4;      // partial sums per lane and part: a_x, a_y,
 // base at or below the stream's lowest index (two per word).  Streams longer than two windows,
 // or spanning more than 65,536 sorted slots, are rebuilt by each pass.
 constexpr uint32_t kLightCacheWords = 2 * 64 + 256;
+// Hit masks of a light item, left by the density pass for the force pass (which then steps
+// through the particles within h only): a word per lane for each (window, row, 32 candidates) in
+// the order both passes walk them.  An item that needs more words is walked in full by both.
+constexpr uint32_t kMaskWords = 6;
 #ifndef FH_PLAN_THREADS
 #define FH_PLAN_THREADS 512
 #endif
@@ -188,10 +192,10 @@ struct fh_ctx {
     uint32_t max_n, max_cells;
     uint32_t max_sort_tiles;
     // sort scratch
-    uint32_t* ka;        // [max_n]
-    uint32_t* va;        // [max_n]
-    uint32_t* kb;        // [max_n]
+    uint32_t* ka;        // [max_n], then va and vb in the same allocation (a HitPlanes plane
+    uint32_t* va;        // [max_n] between the density and the force pass)
     uint32_t* vb;        // [max_n]
+    uint32_t* kb;        // [max_n]
     uint32_t* sort_lb;   // [max_sort_tiles * kDigitSlots] 32-bit look-back words (pass-major)
     uint32_t* hist_part; // [kHistBlocks][kDigitSlots] per-block digit histograms
     uint32_t* sort_pre;  // first-pass tile prefixes of small sorts (tiles of pre_rows_per_tile
@@ -223,6 +227,7 @@ struct fh_ctx {
                          // the force pass
     uint2* lstream_t;    // [3 * ceil(max_n / 64)] stream length of each light item and its lowest
                          // sorted index (~0u: the stream is not kept)
+    uint32_t* hits;      // [3][max_n] the last of a light item's hit mask words (HitPlanes)
     uint64_t* cell_grp;  // [max_cells] epoch << 32 | number of co-located leading particles
     uint2* big;          // [ceil(max_n / 64) + 1] (first slot, sample offset) of group cells
     uint32_t* skip_tag;  // [ceil(max_n / 64)] epoch of the rebuild whose sub-tile holds only group members
@@ -434,7 +439,8 @@ hipError_t launch_csr_from_sorted(fh_ctx* c, const uint32_t* keys, uint32_t n, u
                                   uint32_t* cell_start);
 hipError_t launch_pack_frame(fh_ctx* c, const float* px, const float* py, const float* pz,
                              uint32_t n, uint32_t frame, uint32_t* counter, void* out);
-hipError_t launch_density_fast(fh_ctx* c, const SphArgs& a, const uint32_t* cell_start);
+// `masks`: also leave the light items' hit masks, which launch_force_fast needs.
+hipError_t launch_density_fast(fh_ctx* c, const SphArgs& a, const uint32_t* cell_start, bool masks);
 hipError_t launch_force_fast(fh_ctx* c, const SphArgs& a, const uint32_t* cell_start);
 // Force records of every sorted particle (positions with pressure, velocity and weight over
 // density; density in srho) from the density partials; written into c->sout, which holds the

@@ -108,9 +108,17 @@ constexpr uint32_t kSmallHeavyWork = 32;  // the default below kSmallSystemN par
 constexpr uint32_t kCutFlag = 1u << 31;  // heavy list entry: the item touches a co-located group
 constexpr uint32_t kTransFlag = 1u << 30;  // heavy list entry: walked transposed
 constexpr uint32_t kEntryFlags = kCutFlag | kTransFlag;
-// Item flags (the plan): light (one wavefront), heavy (heavy list), every particle co-located
-// (skipped by both passes).
-constexpr uint8_t kItemLight = 0, kItemHeavy = 1, kItemSkip = 2;
+// Item flags (the plan): light (one wavefront), heavy (heavy list), light with hit masks.
+constexpr uint8_t kItemLight = 0, kItemHeavy = 1, kItemHits = 2;
+// A light item whose largest particle faces at least this many candidates in its slab gets hit
+// masks, so that the force pass steps through the particles within h only (33 of 216 candidates in
+// a dam-break block of 1,048,576 particles: force pass 130 -> 77 us, density pass 61 -> 69 us).  Below,
+// the rows are so short that the masks cost what they save (particles burst onto the walls of the
+// box: passes of 148 + 84 us with every threshold from 32 up, 157 + 95 us with masks for every item).
+#ifndef FH_HITS_MIN
+#define FH_HITS_MIN 48
+#endif
+constexpr uint32_t kHitsMin = FH_HITS_MIN;
 // hslot[item]: the heavy list slot of a heavy item (where its partial sums are), else kNoSlot.
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 // Partial-sum slot of the heavy entry at position pos of sub-list k: the lists interleaved, so a
@@ -631,6 +639,7 @@ __device__ __forceinline__ void plan_work(uint32_t bid, const uint32_t* __restri
                 bool trans = direct_mode == 2u;
                 LightStream L;
                 L.T = ~0u;  // no stream built
+                bool hits = false;
                 if (direct_mode == 1u) {
                     // a light item only when its stream is far longer (pathologically
                     // disjoint ranges: one window would serve one lane at a time); the stream
@@ -640,6 +649,10 @@ __device__ __forceinline__ void plan_work(uint32_t bid, const uint32_t* __restri
                     const uint32_t T = build ? L.T : stream_total(b, e, home_row(ci, g), live, lane);
                     trans = hv ? T > kTransRatio * w + kTransOffset
                                : T > kTransLightRatio * w + kTransLightOffset;
+                    // hit masks: rows of at most 32 candidates in at most two windows are at
+                    // most kMaskWords words
+                    hits = w >= kHitsMin && T <= 2u * kWin &&
+                           __ballot(max(max(e[0] - b[0], e[1] - b[1]), e[2] - b[2]) > 32u) == 0ull;
                 }
                 hv = hv || trans;
                 const uint32_t item = sub * 3u + (uint32_t)slab;
@@ -657,7 +670,7 @@ __device__ __forceinline__ void plan_work(uint32_t bid, const uint32_t* __restri
                 }
                 if (lane == 0) {
                     lstream_t[item] = make_uint2(hv ? ~0u : L.T, base);
-                    flag[item] = hv ? kItemHeavy : kItemLight;
+                    flag[item] = hv ? kItemHeavy : (hits ? kItemHits : kItemLight);
                     if (!hv) hslot[item] = kNoSlot;
                     if (hv)
                         s_item[wave * 3 + (int)nh] =
@@ -810,24 +823,110 @@ __device__ __forceinline__ int next_row(const uint32_t lo[3], const uint32_t hi[
 
 static_assert(kLightCacheWords == kLightHead + kWin, "light stream cache layout");
 
+// Light items stage a window as x, y, z, 12 bytes per candidate.  Their rows are bound by the LDS,
+// and lanes of different cells read about a cell's worth of candidates apart: at 16 bytes a fluid
+// of eight particles per cell puts those reads 128 bytes apart, on the same banks (16.8 LDS cycles
+// per candidate, 8.8 of them conflicts).  1,048,576 particles of a dam-break block: density pass
+// 115 -> 61 us (69 with the hit masks below); a sparse state is unchanged.
+constexpr int kPad = 4;  // candidates of readable LDS behind a window
+
+// The sums of a row in walking order: four candidates in turn, a remainder into the first.
+struct RowSum {
+    float a0, a1, a2, a3;
+    __device__ __forceinline__ float total() const { return (a0 + a1) + (a2 + a3); }
+};
+__device__ __forceinline__ float density_d(const float* __restrict__ q, const float4& pi, float h2) {
+    const float dx = pi.x - q[0], dy = pi.y - q[1], dz = pi.z - q[2];
+    return fmaf(-dz, dz, fmaf(-dy, dy, fmaf(-dx, dx, h2)));
+}
+__device__ __forceinline__ void density_add(float d, float& a) {
+    const float w = fmaxf(d, 0.0f);
+    a = fmaf(w * w, w, a);
+}
+
+// m candidates from p on.
+__device__ __forceinline__ void density_row(const float* __restrict__ p, uint32_t m,
+                                            const float4& pi, float h2, RowSum& S) {
+    const float* const pu = p + 3u * (m & ~3u);
+    const float* const pe = p + 3u * m;
+    while (p < pu) {
+        density_add(density_d(p, pi, h2), S.a0);
+        density_add(density_d(p + 3, pi, h2), S.a1);
+        density_add(density_d(p + 6, pi, h2), S.a2);
+        density_add(density_d(p + 9, pi, h2), S.a3);
+        p += 12;
+    }
+    for (; p < pe; p += 3) density_add(density_d(p, pi, h2), S.a0);
+}
+
+// The same for 1..32 candidates, and which of them lie within h as a bit mask (candidate t at bit
+// 31 - t), from the sign of h^2 - r^2 (one v_alignbit per candidate).  The remainder is one masked
+// step (its reads may run up to two candidates past the lane's, never past the buffer's pad).
+__device__ __forceinline__ uint32_t density_hits(const float* __restrict__ p, uint32_t m,
+                                                 const float4& pi, float h2, RowSum& S) {
+    uint32_t miss = 0;
+    const auto pair = [&](const float* q, bool on, float& a) {
+        const float d = density_d(q, pi, h2);
+        miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(d), 31);
+        density_add(on ? d : 0.0f, a);
+    };
+    const float* const pu = p + 3u * (m & ~3u);
+    while (p < pu) {
+        pair(p, true, S.a0);
+        pair(p + 3, true, S.a1);
+        pair(p + 6, true, S.a2);
+        pair(p + 9, true, S.a3);
+        p += 12;
+    }
+    const uint32_t rest = m & 3u;
+    if (rest) {
+        pair(p, true, S.a0);
+        pair(p + 3, rest > 1u, S.a0);
+        pair(p + 6, rest > 2u, S.a0);
+        miss <<= 1;
+    }
+    // miss holds the last ceil(m / 4) * 4 candidates' bits, first candidate highest
+    const uint32_t hits = ~miss << ((0u - m) & 28u);
+    return hits & ~(0x7FFFFFFFu >> (m - 1u));
+}
+
+// Where the hit mask words of particle s in a slab are, between the density and the force pass:
+// planes that nothing else uses then, so that the masks cost 12 bytes of scratch per particle
+// instead of 72.  Words 0..2 lie where the force pass will write the same (particle, slab)'s three
+// acceleration partials (by the wave that has read the masks), word 3 in the sort's ping-pong
+// buffers, word 4 in the accelerations' part of sout (written by k_finalize), word 5 in hits.
+struct HitPlanes {
+    uint32_t* f;             // fpart
+    uint32_t *w3, *w4, *w5;  // [3][stride] each
+    uint32_t stride;
+};
+__device__ __forceinline__ uint32_t* hit_word(const HitPlanes& H, uint32_t slab, uint32_t q) {
+    // (selects: an indexed member would put the argument into scratch memory)
+    uint32_t* const p = q < 3u ? H.f : (q == 3u ? H.w3 : (q == 4u ? H.w4 : H.w5));
+    return p + (size_t)(q < 3u ? slab * 3u + q : slab) * H.stride;
+}
+
 // Density partials: dpart[slab][s] = sum over the slab's neighbours j of (h^2 - r^2)^3, r^2 < h^2.
 // Light items hold no co-located group (the plan sends those to the heavy list).
+// MASKED: also leave the hit masks (a path of its own: both in one loop cost the unmasked items 10 %).
+template <bool MASKED>
 __device__ __forceinline__ void density_light(uint32_t item, int lane, float4* buf,
                                               const float4* __restrict__ spos,
                                               const uint32_t* __restrict__ skeys, uint32_t n,
                                               GridDesc g, const uint32_t* __restrict__ cstart,
                                               float h2, float* __restrict__ dpart,
-                                              uint32_t stride, uint32_t items,
-                                              const uint8_t* __restrict__ flag,
+                                              uint32_t stride,
                                               const uint32_t* __restrict__ skip_tag,
                                               const Control* __restrict__ ctl,
                                               uint32_t* __restrict__ lstream,
-                                              uint2* __restrict__ lstream_t) {
-    if (item >= items || flag[item] != kItemLight) return;  // whole wave
+                                              uint2* __restrict__ lstream_t,
+                                              const HitPlanes& hits) {
     const uint32_t sub = item / 3u, slab = item - 3u * (item / 3u);
     if (skip_tag[sub] == ctl->epoch) return;  // only group members (finished from the group)
     const uint32_t s = sub * kSub + (uint32_t)lane;
     const bool in = s < n;
+    float* const xyz = (float*)buf;  // the window, 12 bytes per candidate
+    uint32_t words = 0;
     const float4 pi = load_or(spos, s, in, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     // the candidate stream the plan built (short streams), else built here and, when short,
     // kept for the force pass (kLightCacheWords)
@@ -868,13 +967,32 @@ __device__ __forceinline__ void density_light(uint32_t item, int lane, float4* b
         for (int k = 0; k < kWinLoads; k++) v[k] = spos[j[k]];
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int k = 0; k < kWinLoads; k++) buf[k * kWave + lane] = v[k];
+        for (int k = 0; k < kWinLoads; k++) {
+            float* const o = xyz + 3 * (k * kWave + lane);
+            o[0] = v[k].x;
+            o[1] = v[k].y;
+            o[2] = v[k].z;
+        }
         __builtin_amdgcn_wave_barrier();
         uint32_t jb[3], je[3];
         window_rows(L, w0, jb, je);
 #pragma unroll
-        for (int r = 0; r < 3; r++)
-            if (jb[r] < je[r]) acc = density_run(buf, w0, jb[r], je[r], pi, h2, acc);
+        for (int r = 0; r < 3; r++) {
+            const uint32_t m = je[r] - jb[r];
+            const float* const p = xyz + 3u * (jb[r] - w0);
+            RowSum S = {0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (MASKED) {
+                for (uint32_t c = 0; __ballot(c < m) != 0ull; c += 32u) {  // uniform
+                    uint32_t word = 0;
+                    if (c < m) word = density_hits(p + 3u * c, min(m - c, 32u), pi, h2, S);
+                    if (in) hit_word(hits, slab, words)[s] = word;
+                    words++;
+                }
+            } else if (m) {
+                density_row(p, m, pi, h2, S);
+            }
+            acc += S.total();
+        }
     }
     if (in) dpart[(size_t)slab * stride + s] = acc;
 }
@@ -1200,9 +1318,10 @@ void k_density_pass(
     const uint32_t* __restrict__ skip_tag, const Control* __restrict__ ctl,
     uint32_t* __restrict__ lstream, uint2* __restrict__ lstream_t,
     const uint32_t* __restrict__ heavy, uint32_t heavy_cap, float* __restrict__ hpart,
-    uint32_t hgrid, uint32_t hslot_cap) {
+    uint32_t hgrid, uint32_t hslot_cap, HitPlanes hits) {
     constexpr uint32_t hw = HW;
     __shared__ float4 s_p[kWin];
+    static_assert(sizeof(s_p) >= (kWin + kPad) * 3u * sizeof(float), "packed window and its pad");
     const int lane = threadIdx.x;
     const uint32_t b = blockIdx.x, hparts = hgrid * hw;
     if (b < hparts) {  // uniform
@@ -1248,8 +1367,14 @@ void k_density_pass(
         return;
     }
     const uint32_t nl = gridDim.x - hparts;
-    density_light(xcd_chunked(b - hparts, nl), lane, s_p, spos, skeys, n, g, cstart, h2,
-                  dpart, stride, items, flag, skip_tag, ctl, lstream, lstream_t);
+    const uint32_t item = xcd_chunked(b - hparts, nl);
+    const uint8_t kind = item < items ? flag[item] : kItemHeavy;  // uniform
+    if (kind == kItemHits && hits.f)
+        density_light<true>(item, lane, s_p, spos, skeys, n, g, cstart, h2, dpart, stride,
+                            skip_tag, ctl, lstream, lstream_t, hits);
+    else if (kind != kItemHeavy)
+        density_light<false>(item, lane, s_p, spos, skeys, n, g, cstart, h2, dpart, stride,
+                             skip_tag, ctl, lstream, lstream_t, hits);
 }
 
 // A slab partial of particle j: written to its plane (`plane`, already offset to the slab and
@@ -1338,25 +1463,44 @@ __global__ __launch_bounds__(256) void k_prep(const float4* __restrict__ spos,
 // candidates issue ahead of the arithmetic; staged positions are finite (k_prep) and the
 // pressure factor is selected after its product, so a non-pair (r = 0 included) adds exact zeros.
 __device__ __forceinline__ void force_pair(const float4& q, const float4& w, const float4& pi,
-                                           float p_i, const FastForce& K, float& ax, float& ay,
+                                           float p_i, float h, float h2, float& ax, float& ay,
                                            float& az, float& wa) {
     const float dx = pi.x - q.x, dy = pi.y - q.y, dz = pi.z - q.z;
     // r^2 + 1e-30: identical for every pair that passes the test (r^2 > 1e-12), and never 0, so
     // 1/r stays finite and a rejected pair's zeroed (h - r) zeroes its pressure factor as well
     // (one select instead of two)
     const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, 1e-30f)));
-    const bool ok = r2 < K.h2 && r2 > 1e-12f;
+    const bool ok = r2 < h2 && r2 > 1e-12f;
     // The empty asm pins 1/r as computed for every candidate: otherwise the compiler moves the
     // reciprocal square root and the products behind a divergent branch on the pair test, whose
     // exec-mask bookkeeping costs more than the select (10% of the light force work on c3).
     float rinv = __builtin_amdgcn_rsqf(r2);
     asm volatile("" : "+v"(rinv));
-    const float vs = ok ? fmaf(-r2, rinv, K.h) : 0.0f;
+    const float vs = ok ? fmaf(-r2, rinv, h) : 0.0f;
     const float fs = (fmaf(p_i, w.w, q.w) * vs) * (vs * rinv);
     wa = fmaf(vs, w.w, wa);
     ax = fmaf(vs, w.x, fmaf(fs, dx, ax));
     ay = fmaf(vs, w.y, fmaf(fs, dy, ay));
     az = fmaf(vs, w.z, fmaf(fs, dz, az));
+}
+
+// The hits (density_row's mask: candidate t of sp / sv at bit 31 - t) of one lane, two per step
+// with both records' loads in flight; a step's second hit may be missing (the first again, taken
+// with h^2 = 0: adds exact zeros).
+__device__ __forceinline__ void force_hits(const float4* __restrict__ sp,
+                                           const float4* __restrict__ sv, uint32_t hits,
+                                           const float4& pi, float p_i, const FastForce& K,
+                                           float& ax, float& ay, float& az, float& wv) {
+    while (hits) {
+        const int t0 = __builtin_clz(hits);
+        hits ^= 0x80000000u >> t0;
+        const int t1 = hits ? __builtin_clz(hits) : t0;
+        const float h2 = hits ? K.h2 : 0.0f;
+        hits &= ~(0x80000000u >> t1);
+        const float4 q0 = sp[t0], w0 = sv[t0], q1 = sp[t1], w1 = sv[t1];
+        force_pair(q0, w0, pi, p_i, K.h, K.h2, ax, ay, az, wv);
+        force_pair(q1, w1, pi, p_i, K.h, h2, ax, ay, az, wv);
+    }
 }
 
 // U candidates per iteration (their loads issued together).
@@ -1384,13 +1528,13 @@ __device__ __forceinline__ void force_run(const float4* __restrict__ sp,
                     w[u] = v[u];
                 }
 #pragma unroll
-                for (int u = 0; u < U; u++) force_pair(q[u], w[u], pi, p_i, K, ax, ay, az, wv);
+                for (int u = 0; u < U; u++) force_pair(q[u], w[u], pi, p_i, K.h, K.h2, ax, ay, az, wv);
                 p += U;
                 v += U;
             } while (p < pu);
         }
     }
-    for (; p < pe; p++, v++) force_pair(*p, *v, pi, p_i, K, ax, ay, az, wv);
+    for (; p < pe; p++, v++) force_pair(*p, *v, pi, p_i, K.h, K.h2, ax, ay, az, wv);
 }
 
 // Transposed force walk of the item's particles taken by this wave: in the lane of each such
@@ -1423,7 +1567,7 @@ __device__ __forceinline__ void force_trans(const float4* __restrict__ rec,
                     q.w = 0.0f;
                     w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 }
-                force_pair(q, w, pl, pp, K, ax, ay, az, wa);
+                force_pair(q, w, pl, pp, K.h, K.h2, ax, ay, az, wa);
                 j0 = trans_next(j0, j, ok, wb);
             }
         }
@@ -1443,6 +1587,8 @@ __device__ __forceinline__ void force_trans(const float4* __restrict__ rec,
 // Acceleration partials: fpart[slab][c][s] = sum over the slab's neighbours j of the pressure
 // and viscosity pair terms (sph_fused.rs:604-623), not yet divided by rho_i.  Same windowed
 // stream as density_light; the window is staged by copying force records (k_prep).
+// MASKED: the hits of the density pass's masks only.
+template <bool MASKED>
 __device__ __forceinline__ void force_light(uint32_t item, int lane, float4* bp, float4* bv,
                                             const float4* __restrict__ spos,
                                             const float4* __restrict__ svel,
@@ -1450,14 +1596,13 @@ __device__ __forceinline__ void force_light(uint32_t item, int lane, float4* bp,
                                             const float4* __restrict__ rec,
                                             const uint32_t* __restrict__ skeys, uint32_t n,
                                             GridDesc g, const uint32_t* __restrict__ cstart,
-                                            const FastForce& K, float* __restrict__ fpart,
+                                            const FastForce& K, float* fpart,
                                             float* __restrict__ wpart, uint32_t stride,
-                                            uint32_t items, const uint8_t* __restrict__ flag,
                                             const uint32_t* __restrict__ skip_tag,
                                             const Control* __restrict__ ctl,
                                             const uint32_t* __restrict__ lstream,
-                                            const uint2* __restrict__ lstream_t) {
-    if (item >= items || flag[item] != kItemLight) return;  // whole wave
+                                            const uint2* __restrict__ lstream_t,
+                                            const HitPlanes& hits) {
     const uint32_t sub = item / 3u, slab = item - 3u * (item / 3u);
     if (skip_tag[sub] == ctl->epoch) return;  // only group members (finished from the group)
     const uint32_t s = sub * kSub + (uint32_t)lane;
@@ -1473,6 +1618,8 @@ __device__ __forceinline__ void force_light(uint32_t item, int lane, float4* bp,
     const uint2 tb = lstream_t[item];
     L.T = tb.x;
     const bool kept = tb.y != kNoBase;  // uniform
+    // (the next word is loaded ahead)
+    uint32_t word = MASKED && in ? hit_word(hits, slab, 0u)[s] : 0u, words = 0;
     const uint32_t* lc = lstream + (size_t)item * kLightCacheWords;
     if (kept) {
         get_intervals(lc, lane, L);
@@ -1503,9 +1650,21 @@ __device__ __forceinline__ void force_light(uint32_t item, int lane, float4* bp,
             bv[k * kWave + lane] = w[k];
         }
         __builtin_amdgcn_wave_barrier();
-        if (live) {
-            uint32_t jb[3], je[3];
-            window_rows(L, w0, jb, je);
+        uint32_t jb[3], je[3];
+        if (MASKED || live) window_rows(L, w0, jb, je);
+        if constexpr (MASKED) {
+#pragma unroll
+            for (int r = 0; r < 3; r++) {
+                const uint32_t m = je[r] - jb[r];
+                for (uint32_t c = 0; __ballot(c < m) != 0ull; c += 32u) {  // as density_light
+                    const uint32_t now = live && c < m ? word : 0u;
+                    words++;
+                    if (words < kMaskWords && in) word = hit_word(hits, slab, words)[s];
+                    force_hits(bp + (jb[r] - w0 + c), bv + (jb[r] - w0 + c), now, pi, p_i, K, ax,
+                               ay, az, wv);
+                }
+            }
+        } else if (live) {
 #pragma unroll
             for (int r = 0; r < 3; r++)
                 if (jb[r] < je[r]) force_run<4>(bp, bv, w0, jb[r], je[r], pi, p_i, K, ax, ay, az, wv);
@@ -1636,11 +1795,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(6, 8))) v
     const float* __restrict__ srho, const float4* __restrict__ rec,
     const uint32_t* __restrict__ skeys, uint32_t n, GridDesc g,
     const uint32_t* __restrict__ cstart, const uint64_t* __restrict__ cell_grp, FastForce K,
-    float* __restrict__ fpart, float* __restrict__ wpart, uint32_t stride, uint32_t items,
+    float* fpart, float* __restrict__ wpart, uint32_t stride, uint32_t items,
     const uint8_t* __restrict__ flag, const uint32_t* __restrict__ skip_tag,
     const Control* __restrict__ ctl, const uint32_t* __restrict__ lstream,
     const uint2* __restrict__ lstream_t, const uint32_t* __restrict__ heavy,
-    uint32_t heavy_cap, float* __restrict__ hpart, uint32_t hgrid, uint32_t hslot_cap) {
+    uint32_t heavy_cap, float* __restrict__ hpart, uint32_t hgrid, uint32_t hslot_cap,
+    HitPlanes hits) {
     constexpr uint32_t hw = HW;
     __shared__ float4 s_p[kWin];  // x, y, z, p_j
     __shared__ float4 s_v[kWin];  // u/rho_j, w/rho_j
@@ -1698,9 +1858,14 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(6, 8))) v
         return;
     }
     const uint32_t nl = gridDim.x - hparts;
-    force_light(xcd_chunked(b - hparts, nl), lane, s_p, s_v, spos, svel, srho, rec, skeys, n,
-                g, cstart, K, fpart, wpart, stride, items, flag, skip_tag, ctl, lstream,
-                lstream_t);
+    const uint32_t item = xcd_chunked(b - hparts, nl);
+    const uint8_t kind = item < items ? flag[item] : kItemHeavy;  // uniform
+    if (kind == kItemHits)
+        force_light<true>(item, lane, s_p, s_v, spos, svel, srho, rec, skeys, n, g, cstart, K,
+                          fpart, wpart, stride, skip_tag, ctl, lstream, lstream_t, hits);
+    else if (kind != kItemHeavy)
+        force_light<false>(item, lane, s_p, s_v, spos, svel, srho, rec, skeys, n, g, cstart, K,
+                           fpart, wpart, stride, skip_tag, ctl, lstream, lstream_t, hits);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1878,7 +2043,13 @@ hipError_t launch_group_plan(fh_ctx* c, const SphArgs& a, bool with_vel) {
     return hipGetLastError();
 }
 
-hipError_t launch_density_fast(fh_ctx* c, const SphArgs& a, const uint32_t* cell_start) {
+static HitPlanes hit_planes(fh_ctx* c) {
+    return HitPlanes{(uint32_t*)c->fpart, c->ka, (uint32_t*)(c->sout + 2 * (size_t)c->max_n),
+                     c->hits, c->max_n};
+}
+
+hipError_t launch_density_fast(fh_ctx* c, const SphArgs& a, const uint32_t* cell_start,
+                               bool masks) {
     if (a.n == 0) return hipSuccess;
     uint32_t items;
     const uint32_t grid = wave_grid(a.n, &items);
@@ -1893,7 +2064,7 @@ hipError_t launch_density_fast(fh_ctx* c, const SphArgs& a, const uint32_t* cell
     kernel<<<hgrid * hw + grid, kWave, 0, c->stream>>>(
         c->spos, c->skeys, a.n, a.g, cell_start, c->cell_grp, a.h * a.h, c->dpart, c->max_n,
         items, c->heavy_flag, c->skip_tag, c->ctl, c->lstream, c->lstream_t, c->heavy,
-        c->heavy_cap, c->hpart, hgrid, slot_cap(c, hw));
+        c->heavy_cap, c->hpart, hgrid, slot_cap(c, hw), masks ? hit_planes(c) : HitPlanes{});
     hipError_t e = hipGetLastError();
     tend(c, KID_DENSITY);
     return e;
@@ -1943,7 +2114,7 @@ hipError_t launch_force_fast(fh_ctx* c, const SphArgs& a, const uint32_t* cell_s
     kernel<<<hgrid * hw + grid, kWave, 0, c->stream>>>(
         c->spos, c->svel, c->srho, c->sout, c->skeys, a.n, a.g, cell_start, c->cell_grp, K,
         c->fpart, c->wpart, c->max_n, items, c->heavy_flag, c->skip_tag, c->ctl, c->lstream,
-        c->lstream_t, c->heavy, c->heavy_cap, c->hpart, hgrid, slot_cap(c, hw));
+        c->lstream_t, c->heavy, c->heavy_cap, c->hpart, hgrid, slot_cap(c, hw), hit_planes(c));
     hipError_t e = hipGetLastError();
     tend(c, KID_FORCE);
     return e;

@@ -162,6 +162,25 @@ def test_step_with_velocities_matches_oracle(fh, gpu_ctx, oracle, mode):
     print("bit-exact fractions", exact)
 
 
+@pytest.mark.parametrize("per_cell", [5, 8, 10, 11, "mixed"])
+def test_hit_masks_match_oracle(fh, gpu_ctx, oracle, per_cell):
+    """Light items with hit masks, one item per wave: rows of 15, 24, 30 and 33 candidates (a mask
+    word holds 32; an item with a longer row has no masks), streams of one and two windows, and
+    rows of every length beside one another; the bound is the one-step bar of check_step."""
+    from forge_hip import workloads
+    cfg = workloads.small_sph(n=4096)
+    rng = np.random.default_rng(77)
+    cells = np.array([(x, y, z) for z in range(4, 11) for y in range(9) for x in range(3, 33)])
+    k = rng.integers(0, 13, len(cells)) if per_cell == "mixed" else np.full(len(cells), per_cell)
+    p = (np.repeat(cells, k, axis=0) + rng.uniform(0.02, 0.98, (int(k.sum()), 3))) * cfg.cell_size
+    p = p[rng.permutation(len(p))].astype(np.float32)
+    cfg.n = len(p)
+    cfg.x, cfg.y, cfg.z = (np.ascontiguousarray(p[:, a]) for a in range(3))
+    vel = [rng.uniform(-0.5, 0.5, cfg.n).astype(np.float32) for _ in range(3)]
+    print(f"hit masks: {per_cell} per cell, {cfg.n} particles", flush=True)
+    check_step(fh, oracle, cfg, vel, mode="fastlarge")
+
+
 def test_c3_step1_matches_oracle(fh, gpu_ctx, oracle):
     """configs[3] at full size (1,048,576 particles), first substep, fast passes."""
     from forge_hip import workloads
