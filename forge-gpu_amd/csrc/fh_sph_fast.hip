@@ -104,7 +104,15 @@ __device__ __forceinline__ void slab_ranges(const CellXYZ& c, bool live, const G
 // items.  The plan is made once per substep and serves both passes.
 constexpr int kSub = 64;                // particles per sub-tile (one wavefront)
 constexpr uint32_t kHeavyWork = 192;   // default: candidates per particle and slab
-constexpr uint32_t kSmallHeavyWork = 32;  // the default below kSmallSystemN particles
+// The default below kSmallSystemN particles, except for items with hit masks whose stream is at most
+// kSmallHitsT candidates: a fluid at rest faces ~72 candidates per particle and slab, and splitting
+// every such item made each pass many times its work (10 substeps of a dam-break block: 50,000
+// particles 1620 -> 870 us, 10,000 1320 -> 745, 200,000 2760 -> 1240 us).  Longer streams, of several
+// home rows and windows, keep the split: a limit of 256 gave 1150 us for 50,000 particles, 320 and
+// 400 870, 512 905 (particles on the walls of the box: 60,000 in 173-179 us at every limit, 182
+// before; without this rule's heavy items 196-215).
+constexpr uint32_t kSmallHeavyWork = 32;
+constexpr uint32_t kSmallHitsT = 384;
 constexpr uint32_t kCutFlag = 1u << 31;  // heavy list entry: the item touches a co-located group
 constexpr uint32_t kTransFlag = 1u << 30;  // heavy list entry: walked transposed
 constexpr uint32_t kEntryFlags = kCutFlag | kTransFlag;
@@ -606,7 +614,8 @@ __device__ __forceinline__ void plan_work(uint32_t bid, const uint32_t* __restri
                                           const uint64_t* __restrict__ cand_tag,
                                           uint8_t* __restrict__ flag,
                                           uint32_t* __restrict__ heavy, uint32_t heavy_cap,
-                                          uint32_t heavy_work, uint32_t direct_mode,
+                                          uint32_t heavy_work, uint32_t small_work,
+                                          uint32_t direct_mode,
                                           Control* ctl, uint32_t* __restrict__ lstream,
                                           uint2* __restrict__ lstream_t,
                                           uint32_t* __restrict__ hslot, uint32_t hslot_cap) {
@@ -653,6 +662,12 @@ __device__ __forceinline__ void plan_work(uint32_t bid, const uint32_t* __restri
                     // most kMaskWords words
                     hits = w >= kHitsMin && T <= 2u * kWin &&
                            __ballot(max(max(e[0] - b[0], e[1] - b[1]), e[2] - b[2]) > 32u) == 0ull;
+                    if (!hv && small_work && w > small_work && !(hits && T <= kSmallHitsT)) {
+                        hv = true;
+                        trans = T > kTransRatio * w + kTransOffset;
+                    }
+                } else if (small_work && w > small_work) {
+                    hv = true;
                 }
                 hv = hv || trans;
                 const uint32_t item = sub * 3u + (uint32_t)slab;
@@ -720,15 +735,16 @@ __global__ __launch_bounds__(kPlanThreads, 8) void k_group_plan(
     uint32_t* __restrict__ sidx, uint32_t* __restrict__ rank, uint32_t* __restrict__ scratch,
     uint64_t* __restrict__ cell_grp, float4* __restrict__ vrep, uint32_t* __restrict__ skip_tag,
     GridDesc g, const uint64_t* __restrict__ cand_tag, uint8_t* __restrict__ flag,
-    uint32_t* __restrict__ heavy, uint32_t heavy_cap, uint32_t heavy_work, uint32_t direct_mode,
-    Control* ctl, uint32_t* __restrict__ lstream, uint2* __restrict__ lstream_t,
+    uint32_t* __restrict__ heavy, uint32_t heavy_cap, uint32_t heavy_work,
+    uint32_t small_work, uint32_t direct_mode, Control* ctl, uint32_t* __restrict__ lstream, uint2* __restrict__ lstream_t,
     uint32_t* __restrict__ hslot, uint32_t hslot_cap) {
     if (blockIdx.x < kGroupBlocks)
         group_work(blockIdx.x, kGroupBlocks, big, cap, n, skeys, cstart, spos, svel, sidx, rank,
                    scratch, cell_grp, vrep, skip_tag, ctl);
     else
         plan_work(blockIdx.x - kGroupBlocks, skeys, n, g, cstart, cand_tag, flag, heavy,
-                  heavy_cap, heavy_work, direct_mode, ctl, lstream, lstream_t, hslot, hslot_cap);
+                  heavy_cap, heavy_work, small_work, direct_mode, ctl, lstream, lstream_t, hslot,
+                  hslot_cap);
 }
 
 // The heavy work lists of this substep as one sequence: entry q of the concatenation of the
@@ -1287,14 +1303,17 @@ static uint32_t heavy_parts(const fh_ctx* c, uint32_t n) {
     const uint64_t room = (uint64_t)kHeavyLists * c->heavy_cap * c->hpart_parts;
     return n < kSmallSystemN && room >= 8ull * slots_needed(n) ? 8u : (uint32_t)kHeavyWaves;
 }
-// Candidates per particle and slab above which an item is split: FH_OPT_HEAVY_WORK, else 32 for
-// small systems (configs[0]: 120 -> 90 us per substep with 8 parts; 24, 28, 36, 40 gave 102, 96,
-// 92 and 100 us, every item split 195 us) and 192 otherwise (configs[3]'s trajectory: 412.9 ->
-// 406.1 us per substep against 384; 160: 407.8; its fixed state with 96, 128, 224, 256: 418.7,
+// Candidates per particle and slab above which an item is split: FH_OPT_HEAVY_WORK, else 192, and for
+// small systems, except short items with hit masks, 32 (configs[0] burst onto the walls: 120 ->
+// 90 us per substep with 8 parts; 24, 28, 36, 40 gave 102, 96, 92 and 100 us, every item split
+// 195 us; 192: configs[3]'s trajectory 412.9 -> 406.1 us per substep against 384; 160: 407.8; its fixed state with 96, 128, 224, 256: 418.7,
 // 423.5, 410.0, 411.9 us; above 384 a light item's stream no longer fits the two windows kept
 // for the force pass: 512 took 729 us).
-static uint32_t heavy_work(const fh_ctx* c, uint32_t n) {
-    return c->heavy_work ? c->heavy_work : n < kSmallSystemN ? kSmallHeavyWork : kHeavyWork;
+static uint32_t heavy_work(const fh_ctx* c) {
+    return c->heavy_work ? c->heavy_work : kHeavyWork;
+}
+static uint32_t small_work(const fh_ctx* c, uint32_t n) {
+    return !c->heavy_work && n < kSmallSystemN ? kSmallHeavyWork : 0u;
 }
 static uint32_t heavy_grid(uint32_t items) {
     const uint32_t g = (items / 8u + 7u) / 8u * 8u;
@@ -2036,7 +2055,7 @@ hipError_t launch_group_plan(fh_ctx* c, const SphArgs& a, bool with_vel) {
                                 c->spos, with_vel ? c->svel : nullptr, c->sidx, c->rank, c->ka,
                                 c->cell_grp, c->vrep, c->skip_tag, a.g, c->run_tag,
                                 c->heavy_flag, c->heavy, c->heavy_cap,
-                                heavy_work(c, a.n), c->direct_mode,
+                                heavy_work(c), small_work(c, a.n), c->direct_mode,
                                 c->ctl, c->lstream, c->lstream_t, c->hslot,
                                 slot_cap(c, heavy_parts(c, a.n)));
     tend(c, KID_PLAN);

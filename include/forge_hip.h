@@ -271,7 +271,8 @@ int fh_sph_fused_steps(fh_ctx* ctx, const fh_sph_params* prm, const fh_epilogue*
  * particles face more than `value` candidates (a co-located group counting as one) is processed
  * by 4 (or 8: FH_OPT_HEAVY_PARTS) wavefronts that split its candidates instead of one
  * wavefront; value 0 restores the default: 192, or 32 for calls of fewer than 2^18 particles,
- * whose few items would not fill the GPU otherwise.  Results differ only by rounding. */
+ * whose few items would not fill the GPU otherwise (there, items of an even fluid of up to 32
+ * candidates per row stay whole).  Results differ only by rounding. */
 #define FH_OPT_HEAVY_WORK 2
 /* FH_OPT_DIRECT_ITEMS = 3: items whose particles' candidate ranges barely overlap (sparse
  * particles along a row, or beside a dense one) are walked transposed: one particle at a time,

@@ -177,8 +177,9 @@ def test_hit_masks_match_oracle(fh, gpu_ctx, oracle, per_cell):
     cfg.n = len(p)
     cfg.x, cfg.y, cfg.z = (np.ascontiguousarray(p[:, a]) for a in range(3))
     vel = [rng.uniform(-0.5, 0.5, cfg.n).astype(np.float32) for _ in range(3)]
-    print(f"hit masks: {per_cell} per cell, {cfg.n} particles", flush=True)
-    check_step(fh, oracle, cfg, vel, mode="fastlarge")
+    for mode in ("fastlarge", "fast"):  # "fast": short streams whole, the others split
+        print(f"hit masks: {per_cell} per cell, {cfg.n} particles, {mode}", flush=True)
+        check_step(fh, oracle, cfg, vel, mode=mode)
 
 
 def test_c3_step1_matches_oracle(fh, gpu_ctx, oracle):
