@@ -217,10 +217,11 @@ int fh_create(int device, uint32_t max_n, uint32_t max_cells, void* stream, fh_c
     c->max_sort_tiles = ceil_div(max_n, (uint32_t)kSortTile);
     size_t tot = 0;
     hipError_t e = hipSuccess;
-    if (e == hipSuccess) e = alloc(&c->ka, 3 * (size_t)max_n, &tot);
+    c->sort_stride = ceil_div(max_n, 64u) * 64u;
+    if (e == hipSuccess) e = alloc(&c->ka, 3 * (size_t)c->sort_stride, &tot);
     if (e == hipSuccess) {
-        c->va = c->ka + max_n;
-        c->vb = c->ka + 2 * (size_t)max_n;
+        c->va = c->ka + c->sort_stride;
+        c->vb = c->ka + 2 * (size_t)c->sort_stride;
     }
     if (e == hipSuccess) e = alloc(&c->kb, max_n, &tot);
     if (e == hipSuccess) e = alloc(&c->sort_lb, (size_t)c->max_sort_tiles * kDigitSlots, &tot);
@@ -592,7 +593,7 @@ int fh_sph_force(fh_ctx* c, const fh_sph_params* prm, const float* px, const flo
               prm->rest_density, prm->viscosity_coefficient, dt, n};
     // the caller's state in the caller's grid order, then the exact fused pass (velocities
     // written back through sorted_indices; positions untouched without an epilogue)
-    FH_CHECK_HIP(launch_gather_grid(c, px, py, pz, vx, vy, vz, density, sorted_indices, n));
+    FH_CHECK_HIP(launch_gather_grid(c, px, py, pz, vx, vy, vz, density, sorted_indices, n, false));
     FH_CHECK_HIP(launch_force(c, a, nullptr, cell_start, nullptr, nullptr, nullptr, vx, vy, vz,
                               accel));
     return FH_OK;

@@ -192,9 +192,10 @@ struct fh_ctx {
     uint32_t max_n, max_cells;
     uint32_t max_sort_tiles;
     // sort scratch
-    uint32_t* ka;        // [max_n], then va and vb in the same allocation (a HitPlanes plane
-    uint32_t* va;        // [max_n] between the density and the force pass)
+    uint32_t* ka;        // [max_n], then va and vb sort_stride words apart in the same allocation
+    uint32_t* va;        // [max_n] (a HitPlanes plane between the density and the force pass)
     uint32_t* vb;        // [max_n]
+    uint32_t sort_stride; // max_n rounded up to whole 256-byte rows of a wave
     uint32_t* kb;        // [max_n]
     uint32_t* sort_lb;   // [max_sort_tiles * kDigitSlots] 32-bit look-back words (pass-major)
     uint32_t* hist_part; // [kHistBlocks][kDigitSlots] per-block digit histograms
@@ -434,7 +435,8 @@ hipError_t launch_gather(fh_ctx* c, const GridDesc& g, uint32_t cells, const flo
 hipError_t launch_gather_resident(fh_ctx* c, uint32_t cells, uint32_t n);
 hipError_t launch_gather_grid(fh_ctx* c, const float* px, const float* py, const float* pz,
                               const float* vx, const float* vy, const float* vz,
-                              const float* density, const uint32_t* sorted_indices, uint32_t n);
+                              const float* density, const uint32_t* sorted_indices, uint32_t n,
+                              bool skip_bad);
 hipError_t launch_csr_from_sorted(fh_ctx* c, const uint32_t* keys, uint32_t n, uint32_t cells,
                                   uint32_t* cell_start);
 hipError_t launch_pack_frame(fh_ctx* c, const float* px, const float* py, const float* pz,
@@ -466,7 +468,7 @@ hipError_t launch_force(fh_ctx* c, const SphArgs& a, const fh_epilogue* epi,
                         const uint32_t* cell_start, float* px, float* py, float* pz, float* vx,
                         float* vy, float* vz, float* accel);
 // Unfused pressure (viscosity = false) or viscosity pass over a caller grid, updating v in place
-// (the viscosity pass first copies v into c->svel: every neighbour reads the state before it).
+// (the state is first copied to slot order: every neighbour reads the state before the pass).
 hipError_t launch_unfused(fh_ctx* c, bool viscosity, const SphArgs& a, const float* px,
                           const float* py, const float* pz, float* vx, float* vy, float* vz,
                           const float* density, const uint32_t* cell_start,

@@ -14,6 +14,7 @@
 // density and velocity updates reproduce the CPU restatement of sph_density.rs:409-460 and
 // sph_fused.rs:542-638.
 #include "fh_internal.hpp"
+#include "fh_stream.hpp"
 
 namespace fh {
 
@@ -307,20 +308,26 @@ hipError_t launch_csr_from_sorted(fh_ctx* c, const uint32_t* keys, uint32_t n, u
     return hipGetLastError();
 }
 
-// Sorted-order state for the exact force pass over a caller's grid (sorted_indices[s] = the
-// particle in slot s): the same layout k_gather writes, plus the densities.
+// Sorted-order state for the exact passes over a caller's grid (sorted_indices[s] = the particle in
+// slot s): the same layout k_gather writes, plus the densities.  A malformed id is never written
+// back; as a neighbour it reads particle 0 in the force pass, and is none in the unfused passes
+// (SKIP_BAD: a NaN position passes no distance test), which also get rank[i], a slot of particle i.
+template <bool SKIP_BAD>
 __global__ __launch_bounds__(256) void k_gather_grid(
     const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
     const float* __restrict__ vx, const float* __restrict__ vy, const float* __restrict__ vz,
     const float* __restrict__ density, const uint32_t* __restrict__ sorted_indices, uint32_t n,
     float4* __restrict__ spos, float4* __restrict__ svel, float* __restrict__ srho,
-    uint32_t* __restrict__ sidx) {
+    uint32_t* __restrict__ sidx, uint32_t* __restrict__ rank) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
     const uint32_t i = sorted_indices[s];
-    const bool ok = i < n;  // a malformed id reads particle 0 and is never written back
+    const bool ok = i < n;
     const uint32_t q = ok ? i : 0u;
-    spos[s] = make_float4(px[q], py[q], pz[q], __uint_as_float(s));
+    const float bad = __builtin_nanf("");
+    spos[s] = SKIP_BAD && !ok ? make_float4(bad, bad, bad, 0.0f)
+                              : make_float4(px[q], py[q], pz[q], __uint_as_float(s));
+    if (SKIP_BAD && ok) rank[i] = s;
     svel[s] = make_float4(vx[q], vy[q], vz[q], __uint_as_float(q));
     srho[s] = density[q];
     sidx[s] = ok ? i : 0xFFFFFFFFu;
@@ -328,12 +335,14 @@ __global__ __launch_bounds__(256) void k_gather_grid(
 
 hipError_t launch_gather_grid(fh_ctx* c, const float* px, const float* py, const float* pz,
                               const float* vx, const float* vy, const float* vz,
-                              const float* density, const uint32_t* sorted_indices, uint32_t n) {
+                              const float* density, const uint32_t* sorted_indices, uint32_t n,
+                              bool skip_bad) {
     if (n == 0) return hipSuccess;
     tbeg(c, KID_GATHER);
-    k_gather_grid<<<ceil_div(n, 256u), 256, 0, c->stream>>>(px, py, pz, vx, vy, vz, density,
-                                                            sorted_indices, n, c->spos, c->svel,
-                                                            c->srho, c->sidx);
+    const auto kernel = skip_bad ? k_gather_grid<true> : k_gather_grid<false>;
+    kernel<<<ceil_div(n, 256u), 256, 0, c->stream>>>(px, py, pz, vx, vy, vz, density,
+                                                     sorted_indices, n, c->spos, c->svel, c->srho,
+                                                     c->sidx, c->rank);
     tend(c, KID_GATHER);
     return hipGetLastError();
 }
@@ -392,40 +401,208 @@ __device__ __forceinline__ Cell3 sph_cell(const float4& p, const GridDesc& g) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Density: rho_i = sum_j mass*poly6*(h2 - r2)^3 over r2 < h2, self included.
-__global__ __launch_bounds__(256) void k_density(const float4* __restrict__ spos,
-                                                 const uint32_t* __restrict__ sidx, uint32_t n,
-                                                 GridDesc g, const uint32_t* __restrict__ cstart,
-                                                 float h2, float mc, float* __restrict__ srho,
-                                                 float* __restrict__ density) {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const float4 pi = spos[s];
-    const Cell3 c = sph_cell(pi, g);
-    const int x0 = c.cx > 0 ? c.cx - 1 : 0;
-    const int x1 = c.cx + 1 < (int)g.nx ? c.cx + 1 : (int)g.nx - 1;
-    float rho = 0.0f;
-    for (int dz = -1; dz <= 1; dz++) {
-        int nz = c.cz + dz;
-        if (nz < 0 || nz >= (int)g.nz) continue;
-        for (int dy = -1; dy <= 1; dy++) {
-            int ny = c.cy + dy;
-            if (ny < 0 || ny >= (int)g.ny) continue;
-            uint32_t row = (uint32_t)ny * g.nx + (uint32_t)nz * g.nx * g.ny;
-            uint32_t b = cstart[row + (uint32_t)x0], e = min(cstart[row + (uint32_t)x1 + 1u], n);
-            for (uint32_t j = b; j < e; j++) {
-                float4 q = spos[j];
-                float dx2 = pi.x - q.x;
-                float dy2 = pi.y - q.y;
-                float dz2 = pi.z - q.z;
-                float r2 = dx2 * dx2 + dy2 * dy2 + dz2 * dz2;
-                if (r2 < h2) {
-                    float diff = h2 - r2;
-                    rho += mc * diff * diff * diff;
-                }
-            }
+// Neighbour walk of the bit-exact passes: one wave per 64 consecutive sorted particles, each lane
+// visiting its own candidates in the reference's order (dz, dy, dx, then ascending slot).  The
+// candidates are staged through LDS a window at a time (the stream of fh_stream.hpp, one z-slab
+// after the other), 12 bytes of position each, so that a candidate costs the wave three LDS dwords
+// instead of a 16-byte gather per lane.
+//
+// For the passes whose pair terms hold IEEE divisions and square roots (~70 VALU instructions,
+// and one lane in six is within h) a row is walked twice: first the distance test of up to 32
+// candidates into a bit mask per lane, then the set bits.  In one loop every candidate that is a
+// neighbour of any of the 64 lanes costs the whole wave the divisions: 216 times per particle of
+// a dam-break block against ~54, the longest lane's hits.  262,144 particles of such a block: force
+// pass 124 -> 64 us, density pass (one walk) 52 -> 35 us; 400,000: force pass 145 -> 106 us.
+//
+// The stream needs the lanes' ranges to grow along a home row and to be those of a grid built over
+// these positions.  A wave that finds otherwise (a caller's grid of other positions), or whose
+// stream is far longer than its lanes' ranges (sparse particles beside a dense row), walks its
+// lanes' ranges in global memory instead: the same candidates in the same order.
+// 320 candidates per window: 262,144 particles, force pass 64 us (256: 73, 384: 87, 192: 92; each
+// further window is another round of loads, a larger one leaves fewer waves per SIMD).
+constexpr int kExactWin = 320;
+// (64 home rows of 3 unions of at most n candidates each: no 32-bit overflow of a stream's length)
+constexpr uint32_t kExactStreamN = 1u << 24;
+struct ExactLds {
+    float xyz[3 * (kExactWin + 4)];  // (a row's masked last step reads up to 3 candidates past it)
+};
+
+// The three row ranges of slab dz around cell c, clamped to n (empty outside the grid, and where a
+// malformed grid has them inverted).
+__device__ __forceinline__ void exact_ranges(const Cell3& c, bool live, const GridDesc& g,
+                                             const uint32_t* __restrict__ cstart, uint32_t n,
+                                             int dz, uint32_t b[3], uint32_t e[3]) {
+    const uint32_t x0 = (uint32_t)(c.cx > 0 ? c.cx - 1 : 0);
+    const uint32_t x1 = (uint32_t)(c.cx + 1 < (int)g.nx ? c.cx + 1 : (int)g.nx - 1);
+    const int nz = c.cz + dz;
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        const int ny = c.cy + r - 1;
+        b[r] = e[r] = 0u;
+        if (live && nz >= 0 && nz < (int)g.nz && ny >= 0 && ny < (int)g.ny) {
+            const uint32_t row = (uint32_t)ny * g.nx + (uint32_t)nz * g.nx * g.ny;
+            e[r] = min(cstart[row + x1 + 1u], n);
+            b[r] = min(cstart[row + x0], e[r]);
         }
     }
+}
+
+// Whether the wave's ranges can be laid out as a stream (uniform).
+__device__ __forceinline__ bool exact_streams(const uint32_t b[3], const uint32_t e[3],
+                                              uint32_t hr, bool in, int lane) {
+    const uint32_t hp = (uint32_t)__shfl_up((int)hr, 1u, kWave);
+    const bool same = in && lane > 0 && hp == hr;
+    bool ok = !in || lane == 0 || hp <= hr;  // home rows in order: each is one run of lanes
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        const uint32_t bp = (uint32_t)__shfl_up((int)b[r], 1u, kWave);
+        const uint32_t ep = (uint32_t)__shfl_up((int)e[r], 1u, kWave);
+        ok = ok && (!same || (bp <= b[r] && ep <= e[r]));
+    }
+    return __ballot(!ok) == 0ull;
+}
+
+// Walks the neighbourhood of the lanes with `in` (consecutive from lane 0).  load(j): what the pass
+// needs of sorted particle j beside its position (float4), store(slot, v): to window slot `slot`;
+// row(p, w, m): m candidates, positions at p (12 bytes each), at window slot w on;
+// one(j): a candidate in global memory.
+template <class Load, class Store, class Row, class One>
+__device__ __forceinline__ void exact_walk(ExactLds& lds, const float4* __restrict__ spos,
+                                           uint32_t n, const GridDesc& g,
+                                           const uint32_t* __restrict__ cstart, const Cell3& c,
+                                           bool in, int lane, Load&& load, Store&& store,
+                                           Row&& row, One&& one) {
+    const uint32_t hr = (uint32_t)c.cy + (uint32_t)c.cz * g.ny;
+    for (int dz = -1; dz <= 1; dz++) {  // uniform
+        uint32_t b[3], e[3];
+        exact_ranges(c, in, g, cstart, n, dz, b, e);
+        LightStream L;
+        bool stream = n <= kExactStreamN && exact_streams(b, e, hr, in, lane);
+        if (stream) {
+            light_stream(L, b, e, hr, in, lane);
+            const uint32_t w = wave_max(L.cnt[0] + L.cnt[1] + L.cnt[2]);
+            stream = L.T <= 16u * w + 2048u;
+        }
+        if (!stream) {
+#pragma unroll 1
+            for (int r = 0; r < 3; r++)
+                for (uint32_t j = b[r]; j < e[r]; j++) one(j);
+            continue;
+        }
+        for (uint32_t w0 = 0; w0 < L.T; w0 += kExactWin) {  // uniform
+            uint32_t j[kExactWin / kWave];
+            window_indices<kExactWin>(L, w0, lane, j);
+            float4 v[kExactWin / kWave], u[kExactWin / kWave];
+#pragma unroll
+            for (int k = 0; k < kExactWin / kWave; k++) {
+                v[k] = spos[j[k]];
+                u[k] = load(j[k]);
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int k = 0; k < kExactWin / kWave; k++) {
+                float* const o = lds.xyz + 3 * (k * kWave + lane);
+                o[0] = v[k].x;
+                o[1] = v[k].y;
+                o[2] = v[k].z;
+                store(k * kWave + lane, u[k]);
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+            for (int r = 0; r < 3; r++) {  // in the reference's order
+                const uint32_t S = r == 0 ? L.S[0] : (r == 1 ? L.S[1] : L.S[2]);
+                const uint32_t cnt = r == 0 ? L.cnt[0] : (r == 1 ? L.cnt[1] : L.cnt[2]);
+                const uint32_t jb = max(S, w0), je = min(S + cnt, w0 + (uint32_t)kExactWin);
+                const uint32_t m = cnt && je > jb ? je - jb : 0u;
+                row(lds.xyz + 3u * (jb - w0), jb - w0, m);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
+// A candidate's squared distance with the reference's expressions (sph_fused.rs:594-597).
+__device__ __forceinline__ float exact_r2(const float4& pi, float x, float y, float z) {
+    const float djx = pi.x - x, djy = pi.y - y, djz = pi.z - z;
+    return djx * djx + djy * djy + djz * djz;
+}
+
+// Which of m <= 32 candidates may lie within h: bit 31 - t for candidate t, from the sign of
+// r2 - h2 (exact for every finite r2; the hit itself tests r2 again, so a NaN of either sign does
+// no harm).
+__device__ __forceinline__ uint32_t exact_mask(const float* __restrict__ p, uint32_t m,
+                                               const float4& pi, float h2) {
+    uint32_t mask = 0;
+    const auto test = [&](const float* q) {
+        const float d = exact_r2(pi, q[0], q[1], q[2]) - h2;
+        mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(d), 31);
+    };
+    const float* const pe = p + 3u * ((m + 3u) & ~3u);  // (up to 3 candidates past the row)
+    while (p < pe) {
+        test(p);
+        test(p + 3);
+        test(p + 6);
+        test(p + 9);
+        p += 12;
+    }
+    mask <<= (0u - m) & 28u;
+    return m ? mask & ~(0x7FFFFFFFu >> (m - 1u)) : 0u;
+}
+
+// exact_walk's row for the passes with masks: hit(slot, p) for each candidate that may be within
+// h, in order.
+template <class Hit>
+__device__ __forceinline__ void exact_hits(const float* __restrict__ p, uint32_t w, uint32_t m,
+                                           const float4& pi, float h2, Hit&& hit) {
+    for (uint32_t c = 0; __ballot(c < m) != 0ull; c += 32u) {  // uniform
+        uint32_t mask = c < m ? exact_mask(p + 3u * c, min(m - c, 32u), pi, h2) : 0u;
+        while (mask) {
+            const uint32_t t = (uint32_t)__builtin_clz(mask);
+            mask ^= 0x80000000u >> t;
+            hit(w + c + t, p + 3u * (c + t));
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Density: rho_i = sum_j mass*poly6*(h2 - r2)^3 over r2 < h2, self included.
+__global__ __launch_bounds__(kWave) void k_density(const float4* __restrict__ spos,
+                                                   const uint32_t* __restrict__ sidx, uint32_t n,
+                                                   GridDesc g, const uint32_t* __restrict__ cstart,
+                                                   float h2, float mc, float* __restrict__ srho,
+                                                   float* __restrict__ density) {
+    __shared__ ExactLds lds;
+    const int lane = threadIdx.x;
+    const uint32_t s = xcd_chunked(blockIdx.x, gridDim.x) * kWave + (uint32_t)lane;
+    const bool in = s < n;
+    const float4 pi = spos[in ? s : 0u];
+    const Cell3 c = sph_cell(pi, g);
+    float rho = 0.0f;
+    // a candidate beyond h adds +0.0f, which changes no sum (they start at +0 and never become -0)
+    const auto add = [&](float r2) {
+        const float diff = h2 - r2;
+        const float t = mc * diff * diff * diff;
+        rho += r2 < h2 ? t : 0.0f;
+    };
+    exact_walk(
+        lds, spos, n, g, cstart, c, in, lane, [](uint32_t) { return float4{}; },
+        [](int, const float4&) {},
+        [&](const float* p, uint32_t, uint32_t m) {
+            const float* const pu = p + 3u * (m & ~1u);
+            while (p < pu) {
+                const float ra = exact_r2(pi, p[0], p[1], p[2]);
+                const float rb = exact_r2(pi, p[3], p[4], p[5]);
+                add(ra);
+                add(rb);
+                p += 6;
+            }
+            if (m & 1u) add(exact_r2(pi, p[0], p[1], p[2]));
+        },
+        [&](uint32_t j) {
+            const float4 q = spos[j];
+            add(exact_r2(pi, q.x, q.y, q.z));
+        });
+    if (!in) return;
     srho[s] = rho;
     const uint32_t i = sidx[s];
     if (density && i < n) density[i] = rho;
@@ -441,8 +618,8 @@ hipError_t launch_density(fh_ctx* c, const SphArgs& a, const uint32_t* cell_star
     float poly6 = 315.0f / (64.0f * 3.14159265f * h9);
     float mc = a.mass * poly6;
     tbeg(c, KID_DENSITY);
-    k_density<<<ceil_div(a.n, 256u), 256, 0, c->stream>>>(c->spos, c->sidx, a.n, a.g, cell_start,
-                                                          h2, mc, c->srho, density_out);
+    k_density<<<ceil_div(a.n, (uint32_t)kWave), kWave, 0, c->stream>>>(
+        c->spos, c->sidx, a.n, a.g, cell_start, h2, mc, c->srho, density_out);
     tend(c, KID_DENSITY);
     return hipGetLastError();
 }
@@ -458,65 +635,73 @@ struct ForceConsts {
 // Fused pressure + viscosity (sph_fused.rs:542-638) and the optional epilogue: gravity
 // (gravity.rs:33), integrate with its non-finite guard (integrate.rs:23-29) and the box
 // (box_collider.rs:37-46), written back through sidx to the caller's arrays.
-__global__ __launch_bounds__(256) void k_force(const float4* __restrict__ spos,
-                                               const float4* __restrict__ svel,
-                                               const float* __restrict__ srho,
-                                               const uint32_t* __restrict__ sidx, uint32_t n,
-                                               GridDesc g, const uint32_t* __restrict__ cstart,
-                                               ForceConsts K, float* __restrict__ px,
-                                               float* __restrict__ py, float* __restrict__ pz,
-                                               float* __restrict__ vx, float* __restrict__ vy,
-                                               float* __restrict__ vz,
-                                               float* __restrict__ accel) {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const float4 pi = spos[s];
-    const float4 vi = svel[s];
-    const float rho_i = srho[s];
+// (5 waves per SIMD: left to itself the compiler takes 105 registers, for 4)
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_force(const float4* __restrict__ spos,
+                                                 const float4* __restrict__ svel,
+                                                 const float* __restrict__ srho,
+                                                 const uint32_t* __restrict__ sidx, uint32_t n,
+                                                 GridDesc g, const uint32_t* __restrict__ cstart,
+                                                 ForceConsts K, float* __restrict__ px,
+                                                 float* __restrict__ py, float* __restrict__ pz,
+                                                 float* __restrict__ vx, float* __restrict__ vy,
+                                                 float* __restrict__ vz,
+                                                 float* __restrict__ accel) {
+    __shared__ ExactLds lds;
+    __shared__ float4 s_vr[kExactWin];  // velocity and density of the window's candidates
+    const int lane = threadIdx.x;
+    const uint32_t s = xcd_chunked(blockIdx.x, gridDim.x) * kWave + (uint32_t)lane;
+    const bool in = s < n;
+    const float4 pi = spos[in ? s : 0u];
+    const float4 vi = svel[in ? s : 0u];
+    const float rho_i = srho[in ? s : 0u];
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
     float nvx = vi.x, nvy = vi.y, nvz = vi.z;
-    if (!(rho_i < 1e-6f)) {
-        const float p_i = K.k * (rho_i - K.rho0);
-        float pax = 0.0f, pay = 0.0f, paz = 0.0f;
-        float vax = 0.0f, vay = 0.0f, vaz = 0.0f;
-        const Cell3 c = sph_cell(pi, g);
-        const int x0 = c.cx > 0 ? c.cx - 1 : 0;
-        const int x1 = c.cx + 1 < (int)g.nx ? c.cx + 1 : (int)g.nx - 1;
-        for (int dz = -1; dz <= 1; dz++) {
-            int nz = c.cz + dz;
-            if (nz < 0 || nz >= (int)g.nz) continue;
-            for (int dy = -1; dy <= 1; dy++) {
-                int ny = c.cy + dy;
-                if (ny < 0 || ny >= (int)g.ny) continue;
-                uint32_t row = (uint32_t)ny * g.nx + (uint32_t)nz * g.nx * g.ny;
-                uint32_t b = cstart[row + (uint32_t)x0], e = min(cstart[row + (uint32_t)x1 + 1u], n);
-                for (uint32_t j = b; j < e; j++) {
-                    float4 q = spos[j];
-                    float djx = pi.x - q.x;
-                    float djy = pi.y - q.y;
-                    float djz = pi.z - q.z;
-                    float r2 = djx * djx + djy * djy + djz * djz;
-                    if (r2 < K.h2 && r2 > 1e-12f) {
-                        float r = sqrtf(r2);
-                        float rho_j = srho[j];
-                        if (rho_j < 1e-6f) continue;
-                        float diff = K.h - r;
-                        float p_j = K.k * (rho_j - K.rho0);
-                        float grad_scale = K.gcoef * diff * diff / r;
-                        float f_scale = -K.mass * (p_i + p_j) / (2.0f * rho_j) * grad_scale;
-                        pax += f_scale * djx;
-                        pay += f_scale * djy;
-                        paz += f_scale * djz;
-                        float4 vj = svel[j];
-                        float lap = K.lcoef * diff;
-                        float v_scale = K.mu * K.mass / rho_j * lap;
-                        vax += v_scale * (vj.x - vi.x);
-                        vay += v_scale * (vj.y - vi.y);
-                        vaz += v_scale * (vj.z - vi.z);
-                    }
-                }
-            }
+    const bool live = in && !(rho_i < 1e-6f);
+    const float p_i = K.k * (rho_i - K.rho0);
+    float pax = 0.0f, pay = 0.0f, paz = 0.0f;
+    float vax = 0.0f, vay = 0.0f, vaz = 0.0f;
+    const Cell3 c = sph_cell(pi, g);
+    const auto pair = [&](float qx, float qy, float qz, float vjx, float vjy, float vjz,
+                          float rho_j) {
+        float djx = pi.x - qx;
+        float djy = pi.y - qy;
+        float djz = pi.z - qz;
+        float r2 = djx * djx + djy * djy + djz * djz;
+        if (r2 < K.h2 && r2 > 1e-12f && !(rho_j < 1e-6f)) {
+            float r = sqrtf(r2);
+            float diff = K.h - r;
+            float p_j = K.k * (rho_j - K.rho0);
+            float grad_scale = K.gcoef * diff * diff / r;
+            float f_scale = -K.mass * (p_i + p_j) / (2.0f * rho_j) * grad_scale;
+            pax += f_scale * djx;
+            pay += f_scale * djy;
+            paz += f_scale * djz;
+            float lap = K.lcoef * diff;
+            float v_scale = K.mu * K.mass / rho_j * lap;
+            vax += v_scale * (vjx - vi.x);
+            vay += v_scale * (vjy - vi.y);
+            vaz += v_scale * (vjz - vi.z);
         }
+    };
+    exact_walk(
+        lds, spos, n, g, cstart, c, in, lane,
+        [&](uint32_t j) {
+            const float4 v = svel[j];
+            return make_float4(v.x, v.y, v.z, srho[j]);
+        },
+        [&](int slot, const float4& v) { s_vr[slot] = v; },
+        [&](const float* p, uint32_t w, uint32_t m) {
+            exact_hits(p, w, live ? m : 0u, pi, K.h2, [&](uint32_t slot, const float* q) {
+                const float4 v = s_vr[slot];
+                pair(q[0], q[1], q[2], v.x, v.y, v.z, v.w);
+            });
+        },
+        [&](uint32_t j) {
+            const float4 q = spos[j], v = svel[j];
+            if (live) pair(q.x, q.y, q.z, v.x, v.y, v.z, srho[j]);
+        });
+    if (!in) return;
+    if (live) {
         float inv_rho = 1.0f / rho_i;
         ax = (pax + vax) * inv_rho;
         ay = (pay + vay) * inv_rho;
@@ -590,139 +775,120 @@ hipError_t launch_force(fh_ctx* c, const SphArgs& a, const fh_epilogue* epi,
     }
     K.e = epi ? epi->restitution : 0.0f;
     tbeg(c, KID_FORCE);
-    k_force<<<ceil_div(a.n, 256u), 256, 0, c->stream>>>(c->spos, c->svel, c->srho, c->sidx, a.n,
-                                                        a.g, cell_start, K, px, py, pz, vx, vy,
-                                                        vz, accel);
+    k_force<<<ceil_div(a.n, (uint32_t)kWave), kWave, 0, c->stream>>>(
+        c->spos, c->svel, c->srho, c->sidx, a.n, a.g, cell_start, K, px, py, pz, vx, vy, vz, accel);
     tend(c, KID_FORCE);
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------------------------
-// Unfused modules (sph_pressure.rs:28-112, sph_viscosity.rs:27-106): one thread per particle i
-// in original order, neighbours through the caller's grid (cell_start[C+1], sorted_indices[n]
-// left in the FieldSet by the density module), visited cell by cell in the reference's order
-// (dz, dy, dx, then the cell's range), j == i skipped.  The reference expressions are kept term
-// by term (no contraction, IEEE division and square root), so each velocity equals the CPU
-// restatement's bit for bit.  Ranges and ids are clamped to n so a malformed grid cannot read
-// out of bounds.
+// Unfused modules (sph_pressure.rs:28-112, sph_viscosity.rs:27-106) over the caller's grid
+// (cell_start[C+1], sorted_indices[n] left in the FieldSet by the density module), j == i skipped.
+// The state is copied to slot order first (k_gather_grid), so that the walk is the exact passes'
+// (exact_walk) instead of three scattered reads per candidate and lane; 150,001 particles: pressure
+// 115 -> 51 us, viscosity 120 -> 48 us, the copy (7 us each) included.  The reference expressions are kept term by
+// term (no contraction, IEEE division and square root) in the reference's order, so each velocity
+// equals the CPU restatement's bit for bit.  Ranges and ids are clamped to n so a malformed grid
+// cannot read out of bounds; a particle that a malformed grid holds twice is updated from one of
+// its slots, one that it does not hold is walked from its own position.
 struct UnfusedConsts {
     float h, h2, mass, k, rho0, mu, coef, dt;
     uint32_t n;
 };
 
-template <class Pair>
-__device__ __forceinline__ void unfused_walk(const float* __restrict__ px,
-                                             const float* __restrict__ py,
-                                             const float* __restrict__ pz,
-                                             const float* __restrict__ density,
-                                             const uint32_t* __restrict__ cstart,
-                                             const uint32_t* __restrict__ sidx, GridDesc g,
-                                             const UnfusedConsts& K, uint32_t i, float xi,
-                                             float yi, float zi, Pair&& pair) {
-    const int cx = (int)cell_coord(xi, 0.0f, g.cs, g.nx);
-    const int cy = (int)cell_coord(yi, 0.0f, g.cs, g.ny);
-    const int cz = (int)cell_coord(zi, 0.0f, g.cs, g.nz);
-    for (int dz = -1; dz <= 1; dz++) {
-        const int nzz = cz + dz;
-        if (nzz < 0 || nzz >= (int)g.nz) continue;
-        for (int dy = -1; dy <= 1; dy++) {
-            const int nyy = cy + dy;
-            if (nyy < 0 || nyy >= (int)g.ny) continue;
-            for (int dx = -1; dx <= 1; dx++) {
-                const int nxx = cx + dx;
-                if (nxx < 0 || nxx >= (int)g.nx) continue;
-                const uint32_t cell = (uint32_t)nxx + (uint32_t)nyy * g.nx +
-                                      (uint32_t)nzz * g.nx * g.ny;
-                const uint32_t end = min(cstart[cell + 1u], K.n);
-                for (uint32_t s = cstart[cell]; s < end; s++) {
-                    const uint32_t j = sidx[s];
-                    if (j == i || j >= K.n) continue;
-                    float djx = xi - px[j];
-                    float djy = yi - py[j];
-                    float djz = zi - pz[j];
-                    float r2 = djx * djx + djy * djy + djz * djz;
-                    if (r2 < K.h2 && r2 > 1e-12f) {
-                        float r = sqrtf(r2);
-                        float rho_j = density[j];
-                        if (rho_j < 1e-6f) continue;
-                        pair(j, djx, djy, djz, r, rho_j);
-                    }
-                }
+// sph_pressure.rs:34-111 (K.coef = -45 / (pi h^6)) and sph_viscosity.rs:34-105 (K.coef =
+// 45 / (pi h^6)): one pass over the slots, one lane per slot.  Every neighbour's velocity is the
+// copy's, the state before the pass; the particle's own in-place update goes to v.
+template <bool VISC>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_unfused(
+    const float4* __restrict__ spos, const float4* __restrict__ svel,
+    const float* __restrict__ srho, const uint32_t* __restrict__ sidx,
+    const uint32_t* __restrict__ rank, const float* __restrict__ px, const float* __restrict__ py,
+    const float* __restrict__ pz, const float* __restrict__ density, float* __restrict__ vx,
+    float* __restrict__ vy, float* __restrict__ vz, const uint32_t* __restrict__ cstart,
+    GridDesc g, UnfusedConsts K) {
+    __shared__ ExactLds lds;
+    __shared__ float4 s_vr[kExactWin];  // velocity and density of the window's candidates
+    const int lane = threadIdx.x;
+    const uint32_t s = xcd_chunked(blockIdx.x, gridDim.x) * kWave + (uint32_t)lane;
+    const bool in = s < K.n;
+    const uint32_t i = in ? sidx[s] : K.n;
+    // (ranks are those of this call for every particle the grid holds)
+    const bool own = i < K.n && rank[i] == s;
+    float4 pi = spos[in ? s : 0u];
+    float4 vi = svel[in ? s : 0u];
+    float rho_i = srho[in ? s : 0u];
+    float ax = 0.0f, ay = 0.0f, az = 0.0f;
+    float p_i = K.k * (rho_i - K.rho0);
+    const auto pair = [&](float qx, float qy, float qz, float vjx, float vjy, float vjz,
+                          float rho_j) {
+        float djx = pi.x - qx;
+        float djy = pi.y - qy;
+        float djz = pi.z - qz;
+        float r2 = djx * djx + djy * djy + djz * djz;
+        if (r2 < K.h2 && r2 > 1e-12f && !(rho_j < 1e-6f)) {
+            float r = sqrtf(r2);
+            if constexpr (VISC) {
+                float lap = K.coef * (K.h - r);
+                float scale = K.mu * K.mass / rho_j * lap;
+                ax += scale * (vjx - vi.x);
+                ay += scale * (vjy - vi.y);
+                az += scale * (vjz - vi.z);
+            } else {
+                float diff = K.h - r;
+                float p_j = K.k * (rho_j - K.rho0);
+                float grad_scale = K.coef * diff * diff / r;
+                float f_scale = -K.mass * (p_i + p_j) / (2.0f * rho_j) * grad_scale;
+                ax += f_scale * djx;
+                ay += f_scale * djy;
+                az += f_scale * djz;
             }
         }
+    };
+    const auto update = [&](uint32_t t) {
+        vx[t] = vi.x + (ax / rho_i) * K.dt;
+        vy[t] = vi.y + (ay / rho_i) * K.dt;
+        vz[t] = vi.z + (az / rho_i) * K.dt;
+    };
+    const bool live = own && !(rho_i < 1e-6f);
+    exact_walk(
+        lds, spos, K.n, g, cstart, sph_cell(pi, g), in, lane,
+        [&](uint32_t j) {
+            const float4 v = VISC ? svel[j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            return make_float4(v.x, v.y, v.z, srho[j]);
+        },
+        [&](int slot, const float4& v) { s_vr[slot] = v; },
+        [&](const float* p, uint32_t w, uint32_t m) {
+            exact_hits(p, w, live ? m : 0u, pi, K.h2, [&](uint32_t slot, const float* q) {
+                const float4 v = s_vr[slot];
+                pair(q[0], q[1], q[2], v.x, v.y, v.z, v.w);
+            });
+        },
+        [&](uint32_t j) {
+            const float4 q = spos[j], v = svel[j];
+            if (live) pair(q.x, q.y, q.z, v.x, v.y, v.z, srho[j]);
+        });
+    if (live) update(i);
+    // a particle that the grid does not hold (rank[s] is then no slot of it)
+    const uint32_t rs = in ? rank[s] : 0u;
+    if (in && !(rs < K.n && sidx[rs] == s) && !(density[s] < 1e-6f)) {
+        rho_i = density[s];
+        p_i = K.k * (rho_i - K.rho0);
+        pi = make_float4(px[s], py[s], pz[s], 0.0f);
+        vi = make_float4(vx[s], vy[s], vz[s], 0.0f);  // no slot, so no other thread writes them
+        ax = ay = az = 0.0f;
+        const Cell3 c = sph_cell(pi, g);
+        for (int dz = -1; dz <= 1; dz++) {
+            uint32_t b[3], e[3];
+            exact_ranges(c, true, g, cstart, K.n, dz, b, e);
+            for (int r = 0; r < 3; r++)
+                for (uint32_t j = b[r]; j < e[r]; j++) {
+                    const float4 q = spos[j], v = svel[j];
+                    pair(q.x, q.y, q.z, v.x, v.y, v.z, srho[j]);
+                }
+        }
+        update(s);
     }
-}
-
-// sph_pressure.rs:34-111; K.coef = -45 / (pi h^6).  Pressure terms read positions and
-// densities only, so v_i is updated in place.
-__global__ __launch_bounds__(256) void k_pressure(const float* __restrict__ px,
-                                                  const float* __restrict__ py,
-                                                  const float* __restrict__ pz,
-                                                  float* __restrict__ vx, float* __restrict__ vy,
-                                                  float* __restrict__ vz,
-                                                  const float* __restrict__ density,
-                                                  const uint32_t* __restrict__ cstart,
-                                                  const uint32_t* __restrict__ sidx, GridDesc g,
-                                                  UnfusedConsts K) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= K.n) return;
-    const float rho_i = density[i];
-    if (rho_i < 1e-6f) return;
-    const float p_i = K.k * (rho_i - K.rho0);
-    float ax = 0.0f, ay = 0.0f, az = 0.0f;
-    unfused_walk(px, py, pz, density, cstart, sidx, g, K, i, px[i], py[i], pz[i],
-                 [&](uint32_t, float djx, float djy, float djz, float r, float rho_j) {
-                     float diff = K.h - r;
-                     float p_j = K.k * (rho_j - K.rho0);
-                     float grad_scale = K.coef * diff * diff / r;
-                     float f_scale = -K.mass * (p_i + p_j) / (2.0f * rho_j) * grad_scale;
-                     ax += f_scale * djx;
-                     ay += f_scale * djy;
-                     az += f_scale * djz;
-                 });
-    vx[i] += (ax / rho_i) * K.dt;
-    vy[i] += (ay / rho_i) * K.dt;
-    vz[i] += (az / rho_i) * K.dt;
-}
-
-// Velocities before the viscosity pass (particle order), read for every neighbour.
-__global__ __launch_bounds__(256) void k_copy_vel(const float* __restrict__ vx,
-                                                  const float* __restrict__ vy,
-                                                  const float* __restrict__ vz, uint32_t n,
-                                                  float4* __restrict__ v0) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) v0[i] = make_float4(vx[i], vy[i], vz[i], 0.0f);
-}
-
-// sph_viscosity.rs:34-105; K.coef = 45 / (pi h^6).
-__global__ __launch_bounds__(256) void k_viscosity(const float* __restrict__ px,
-                                                   const float* __restrict__ py,
-                                                   const float* __restrict__ pz,
-                                                   const float4* __restrict__ v0,
-                                                   float* __restrict__ vx, float* __restrict__ vy,
-                                                   float* __restrict__ vz,
-                                                   const float* __restrict__ density,
-                                                   const uint32_t* __restrict__ cstart,
-                                                   const uint32_t* __restrict__ sidx, GridDesc g,
-                                                   UnfusedConsts K) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= K.n) return;
-    const float rho_i = density[i];
-    if (rho_i < 1e-6f) return;
-    const float4 vi = v0[i];
-    float ax = 0.0f, ay = 0.0f, az = 0.0f;
-    unfused_walk(px, py, pz, density, cstart, sidx, g, K, i, px[i], py[i], pz[i],
-                 [&](uint32_t j, float, float, float, float r, float rho_j) {
-                     float lap = K.coef * (K.h - r);
-                     float scale = K.mu * K.mass / rho_j * lap;
-                     const float4 vj = v0[j];
-                     ax += scale * (vj.x - vi.x);
-                     ay += scale * (vj.y - vi.y);
-                     az += scale * (vj.z - vi.z);
-                 });
-    vx[i] = vi.x + (ax / rho_i) * K.dt;
-    vy[i] = vi.y + (ay / rho_i) * K.dt;
-    vz[i] = vi.z + (az / rho_i) * K.dt;
 }
 
 hipError_t launch_unfused(fh_ctx* c, bool viscosity, const SphArgs& a, const float* px,
@@ -741,17 +907,13 @@ hipError_t launch_unfused(fh_ctx* c, bool viscosity, const SphArgs& a, const flo
     K.coef = viscosity ? 45.0f / (3.14159265f * h6) : -45.0f / (3.14159265f * h6);
     K.dt = a.dt;
     K.n = a.n;
-    const uint32_t blocks = ceil_div(a.n, 256u);
-    if (!viscosity) {
-        k_pressure<<<blocks, 256, 0, c->stream>>>(px, py, pz, vx, vy, vz, density, cell_start,
-                                                  sorted_indices, a.g, K);
-        return hipGetLastError();
-    }
-    k_copy_vel<<<blocks, 256, 0, c->stream>>>(vx, vy, vz, a.n, c->svel);
-    hipError_t e = hipGetLastError();
+    const hipError_t e = launch_gather_grid(c, px, py, pz, vx, vy, vz, density, sorted_indices, a.n,
+                                            true);
     if (e != hipSuccess) return e;
-    k_viscosity<<<blocks, 256, 0, c->stream>>>(px, py, pz, c->svel, vx, vy, vz, density,
-                                               cell_start, sorted_indices, a.g, K);
+    const auto kernel = viscosity ? k_unfused<true> : k_unfused<false>;
+    kernel<<<ceil_div(a.n, (uint32_t)kWave), kWave, 0, c->stream>>>(
+        c->spos, c->svel, c->srho, c->sidx, c->rank, px, py, pz, density, vx, vy, vz, cell_start,
+        a.g, K);
     return hipGetLastError();
 }
 

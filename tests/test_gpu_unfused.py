@@ -128,3 +128,86 @@ def test_unfused_pipeline_is_bit_exact(fh, gpu_ctx, oracle):
     assert np.array_equal(f.f32_fields["density"].cpu().numpy(), rho)
     for nm, o in zip(("pos_x", "pos_y", "pos_z", "vel_x", "vel_y", "vel_z"), s):
         assert np.array_equal(f.f32_fields[nm].cpu().numpy(), o), nm
+
+
+def shuffled_grid(kind, cfg, oracle, rng):
+    """A grid the exact walks must not take for one of these positions, or that they walk in its
+    edge cases: positions moved since the build, particles missing from it or held twice, ids
+    beyond n, a sparse row beside a dense one (streams far longer than the lanes' ranges)."""
+    if kind == "sparse":
+        k = cfg.n // 2
+        cfg.x[:k] = rng.uniform(0.0, 1.0, k)
+        cfg.y[:k], cfg.z[:k] = rng.uniform(0.1, 0.124, k), rng.uniform(0.2, 0.224, k)
+        cfg.x[k:], cfg.y[k:] = rng.uniform(0.0, 1.0, cfg.n - k), 0.13
+        cfg.z[k:] = 0.21 + 0.3 * (np.arange(cfg.n - k) % 97 > 0)
+    ocs, osi, _ = oracle.hashgrid_build(cfg.x, cfg.y, cfg.z, cfg.cell_size, (0, 0, 0), cfg.dims)
+    if kind == "moved":
+        for a in ("x", "y", "z"):
+            v = getattr(cfg, a)
+            v += rng.uniform(-0.04, 0.04, cfg.n).astype(np.float32)
+    return ocs, osi
+
+
+@pytest.mark.parametrize("which", ["pressure", "viscosity"])
+@pytest.mark.parametrize("kind", ["moved", "sparse"])
+@pytest.mark.parametrize("n", [65, 6000])
+def test_unfused_pass_over_other_grids_is_bit_exact(fh, gpu_ctx, oracle, which, kind, n):
+    from forge_hip import workloads
+    cfg = workloads.small_sph(n=n, cols=16)
+    rng = np.random.default_rng(n + len(kind))
+    ocs, osi = shuffled_grid(kind, cfg, oracle, rng)
+    vel = state(cfg, 4)
+    prm = oracle.sph_params(cfg.h, cfg.cell_size, cfg.dims, cfg.mass, cfg.gas_constant,
+                            cfg.rest_density, cfg.viscosity)
+    rho = oracle.sph_density(prm, cfg.x, cfg.y, cfg.z, ocs, osi)
+    f = fieldset(fh, cfg, vel)
+    f.f32_fields["density"] = dev(rho)
+    f.u32_fields["cell_start"] = fh.from_u32(ocs)
+    f.u32_fields["sorted_indices"] = fh.from_u32(osi)
+    ref = (oracle.sph_pressure if which == "pressure" else oracle.sph_viscosity)(
+        prm, cfg.x, cfg.y, cfg.z, *vel, rho, ocs, osi, cfg.dt)
+    _, p, v = modules(fh, cfg)
+    f.context(cfg.num_cells)
+    torch.cuda.synchronize()
+    (p if which == "pressure" else v).execute(f, cfg.dt)
+    f.context().sync()
+    for c, nm in enumerate(("vel_x", "vel_y", "vel_z")):
+        assert np.array_equal(f.f32_fields[nm].cpu().numpy(), ref[c]), nm
+
+
+@pytest.mark.parametrize("which", ["pressure", "viscosity"])
+def test_unfused_pass_over_a_malformed_grid(fh, gpu_ctx, oracle, which):
+    """Ids beyond n are no neighbours; a particle the grid holds twice is updated once, one that it
+    does not hold (its slot is taken by the duplicate) from its own position: what the CPU
+    restatement computes with the bad slots removed from the neighbour lists."""
+    from forge_hip import workloads
+    cfg = workloads.small_sph(n=5000, cols=16)
+    vel = state(cfg, 5)
+    ocs, osi, _ = oracle.hashgrid_build(cfg.x, cfg.y, cfg.z, cfg.cell_size, (0, 0, 0), cfg.dims)
+    prm = oracle.sph_params(cfg.h, cfg.cell_size, cfg.dims, cfg.mass, cfg.gas_constant,
+                            cfg.rest_density, cfg.viscosity)
+    rho = oracle.sph_density(prm, cfg.x, cfg.y, cfg.z, ocs, osi)
+    bad = osi.copy()
+    bad[100::500] = 0xFFFFFFF0
+    gone = osi[100::500]
+    # the restatement over the same lists: a particle far away in the place of the missing ids
+    far = cfg.n
+    x, y, z = (np.append(a, np.float32(9.0)) for a in (cfg.x, cfg.y, cfg.z))
+    ids = np.where(bad < cfg.n, bad, far).astype(np.uint32)
+    ov = [np.append(a, np.float32(0.0)) for a in vel]
+    ref = (oracle.sph_pressure if which == "pressure" else oracle.sph_viscosity)(
+        prm, x, y, z, *ov, np.append(rho, np.float32(1.0)), ocs, np.append(ids, np.uint32(far)),
+        cfg.dt)
+    f = fieldset(fh, cfg, vel)
+    f.f32_fields["density"] = dev(rho)
+    f.u32_fields["cell_start"] = fh.from_u32(ocs)
+    f.u32_fields["sorted_indices"] = fh.from_u32(bad)
+    _, p, v = modules(fh, cfg)
+    f.context(cfg.num_cells)
+    torch.cuda.synchronize()
+    (p if which == "pressure" else v).execute(f, cfg.dt)
+    f.context().sync()
+    for c, nm in enumerate(("vel_x", "vel_y", "vel_z")):
+        got = f.f32_fields[nm].cpu().numpy()
+        assert np.array_equal(got, ref[c][:cfg.n]), nm
+    assert not np.array_equal(ref[0][gone], vel[0][gone])  # the missing ones moved as well
