@@ -223,8 +223,47 @@ __global__ __launch_bounds__(kWave) void k_nbr_stream(const float4* __restrict__
     if (wsum) wsum[i] = w;
 }
 
-// Batched HashGrid::query_neighbors: one thread per query, neighbour positions read through
-// sorted_indices from the caller's arrays exactly like hashgrid.rs:176-186.
+// Batched HashGrid::query_neighbors (hashgrid.rs:145-193): kQueryLanes lanes per query walk its nine
+// row ranges together, kQueryStep * kQueryLanes candidates per step with all their loads in
+// flight, and a ballot gives each neighbour its place, so the list keeps the reference's order.
+// Eight lanes, two steps at a time: a row of ~21 candidates (30 neighbours within the radius) takes two.
+//
+// Positions come from a copy in slot order when the batch is large (k_sort_pos), where a row is a few
+// contiguous lines; read through sorted_indices from the caller's arrays every candidate is a line
+// (two more in three separate arrays), and a lane per query waits for them one after the other.
+// 120,000 queries in 600,000 points: 333 us for a count or fill pass with a lane per query, 83 us
+// with eight, the copy (11 us) included; 4, 16 and 32 lanes 110, 82 and 80, and 94 with 16-byte
+// positions: the rows' lines, which mostly miss a 4 MB L2, are what is left.  The copy pays from about
+// one query per hundred points: batches of at least a 32nd of the points make it, and below kQueryCopyMin queries the
+// extra launch would cost more than it gives.  The points' number is the grid's own
+// (cell_start[C]), read on the device; a grid of more points than the context holds is read in place.
+constexpr uint32_t kQueryLanes = 8, kQueryStep = 2, kQueryCopyMin = 1024, kQueryCopyShare = 32;
+struct Pos3 {  // 12 bytes: a row of the copy is a quarter fewer lines than with float4
+    float x, y, z;
+};
+struct QueryCopy {
+    Pos3* spos;      // null: no copy
+    uint32_t max_n;  // its room
+    uint32_t nq;     // queries of the whole batch
+};
+__device__ __forceinline__ bool query_copied(const QueryCopy& Q, uint32_t n) {
+    return Q.spos && n <= Q.max_n && (uint64_t)Q.nq * kQueryCopyShare >= n;
+}
+
+__global__ __launch_bounds__(256) void k_sort_pos(const float* __restrict__ x,
+                                                  const float* __restrict__ y,
+                                                  const float* __restrict__ z, uint32_t stride,
+                                                  const uint32_t* __restrict__ cstart, uint32_t C,
+                                                  const uint32_t* __restrict__ sidx,
+                                                  QueryCopy Q) {
+    const uint32_t n = cstart[C];
+    if (!query_copied(Q, n)) return;
+    for (uint32_t s = blockIdx.x * 256u + threadIdx.x; s < n; s += gridDim.x * 256u) {
+        const size_t o = (size_t)sidx[s] * stride;
+        Q.spos[s] = Pos3{x[o], y[o], z[o]};
+    }
+}
+
 __global__ __launch_bounds__(256) void k_query(const float* __restrict__ x,
                                                const float* __restrict__ y,
                                                const float* __restrict__ z, uint32_t stride,
@@ -236,42 +275,71 @@ __global__ __launch_bounds__(256) void k_query(const float* __restrict__ x,
                                                uint32_t nq, float radius_sq,
                                                uint32_t* __restrict__ counts,
                                                const uint32_t* __restrict__ offsets,
-                                               uint32_t* __restrict__ indices) {
-    uint32_t qi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (qi >= nq) return;
-    size_t oq = (size_t)qi * qstride;
+                                               uint32_t* __restrict__ indices, QueryCopy Q) {
+    const uint32_t t = threadIdx.x % kQueryLanes;
+    const uint32_t shift = (threadIdx.x & 63u) & ~(kQueryLanes - 1u);
+    const uint32_t qi = (blockIdx.x * 256u + threadIdx.x) / kQueryLanes;
+    if (qi >= nq) return;  // whole groups
+    const uint32_t n = cstart[g.nx * g.ny * g.nz];
+    const bool copied = query_copied(Q, n);  // uniform
+    const size_t oq = (size_t)qi * qstride;
     const float px = qx[oq], py = qy[oq], pz = qz[oq];
     const int64_t cx = rust_as_i32(floorf((px - g.ox) / g.cs));
     const int64_t cy = rust_as_i32(floorf((py - g.oy) / g.cs));
     const int64_t cz = rust_as_i32(floorf((pz - g.oz) / g.cs));
     const int64_t x0 = cx - 1 < 0 ? 0 : cx - 1;
     const int64_t x1 = cx + 1 > (int64_t)g.nx - 1 ? (int64_t)g.nx - 1 : cx + 1;
+    // row r = (dz + 1) * 3 + dy + 1 of the reference's walk: lane t loads row t's range, lane 0
+    // also the last one's
+    const auto range = [&](uint32_t r, uint32_t& b, uint32_t& e) {
+        const int64_t nz = cz + (int64_t)(r / 3u) - 1, ny = cy + (int64_t)(r % 3u) - 1;
+        b = e = 0u;
+        if (nz < 0 || nz >= (int64_t)g.nz || ny < 0 || ny >= (int64_t)g.ny || x0 > x1) return;
+        const uint32_t row = (uint32_t)ny * g.nx + (uint32_t)nz * g.nx * g.ny;
+        e = min(cstart[row + (uint32_t)x1 + 1u], n);
+        b = cstart[row + (uint32_t)x0];
+    };
+    uint32_t b0, e0, b8, e8;
+    range(t, b0, e0);
+    range(8u, b8, e8);
     uint32_t cnt = 0;
     uint32_t* out = (offsets && indices) ? indices + offsets[qi] : nullptr;
     const uint32_t room = out ? offsets[qi + 1] - offsets[qi] : 0u;
-    for (int dz = -1; dz <= 1; dz++) {
-        int64_t nz = cz + dz;
-        if (nz < 0 || nz >= (int64_t)g.nz) continue;
-        for (int dy = -1; dy <= 1; dy++) {
-            int64_t ny = cy + dy;
-            if (ny < 0 || ny >= (int64_t)g.ny) continue;
-            if (x0 > x1) continue;
-            uint32_t row = (uint32_t)ny * g.nx + (uint32_t)nz * g.nx * g.ny;
-            uint32_t b = cstart[row + (uint32_t)x0];
-            uint32_t e = cstart[row + (uint32_t)x1 + 1u];
-            for (uint32_t j = b; j < e; j++) {
-                uint32_t pi = sidx[j];
-                size_t o = (size_t)pi * stride;
-                float dx = x[o] - px, dy2 = y[o] - py, dz2 = z[o] - pz;
-                float dist_sq = dx * dx + dy2 * dy2 + dz2 * dz2;
-                if (dist_sq <= radius_sq) {
-                    if (cnt < room) out[cnt] = pi;
-                    cnt++;
+    for (uint32_t r = 0; r < 9u; r++) {
+        const uint32_t b = r < 8u ? (uint32_t)__shfl((int)b0, (int)r, (int)kQueryLanes) : b8;
+        const uint32_t e = r < 8u ? (uint32_t)__shfl((int)e0, (int)r, (int)kQueryLanes) : e8;
+        for (uint32_t j0 = b; j0 < e; j0 += kQueryStep * kQueryLanes) {  // uniform in the group
+            float X[kQueryStep], Y[kQueryStep], Z[kQueryStep];
+#pragma unroll
+            for (uint32_t k = 0; k < kQueryStep; k++) {
+                const uint32_t j = min(j0 + k * kQueryLanes + t, e - 1u);
+                if (copied) {
+                    const Pos3 p = Q.spos[j];
+                    X[k] = p.x;
+                    Y[k] = p.y;
+                    Z[k] = p.z;
+                } else {
+                    const size_t o = (size_t)sidx[j] * stride;
+                    X[k] = x[o];
+                    Y[k] = y[o];
+                    Z[k] = z[o];
                 }
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kQueryStep; k++) {
+                const uint32_t j = j0 + k * kQueryLanes + t;
+                const float dx = X[k] - px, dy2 = Y[k] - py, dz2 = Z[k] - pz;
+                const float dist_sq = dx * dx + dy2 * dy2 + dz2 * dz2;
+                const bool hit = j < e && dist_sq <= radius_sq;
+                const uint32_t m =
+                    (uint32_t)(__ballot(hit) >> shift) & ((1u << kQueryLanes) - 1u);
+                const uint32_t at = cnt + (uint32_t)__popc(m & ((1u << t) - 1u));
+                if (hit && at < room) out[at] = sidx[j];
+                cnt += (uint32_t)__popc(m);
             }
         }
     }
-    counts[qi] = cnt;
+    if (t == 0u) counts[qi] = cnt;
 }
 
 hipError_t launch_query(fh_ctx* c, const float* x, const float* y, const float* z,
@@ -280,10 +348,25 @@ hipError_t launch_query(fh_ctx* c, const float* x, const float* y, const float* 
                         const float* qz, uint32_t qstride, uint32_t nq, float radius,
                         uint32_t* counts, const uint32_t* offsets, uint32_t* indices) {
     if (nq == 0) return hipSuccess;
-    k_query<<<ceil_div(nq, 256u), 256, 0, c->stream>>>(x, y, z, stride, g, cell_start,
-                                                       sorted_indices, qx, qy, qz, qstride, nq,
-                                                       radius * radius, counts, offsets, indices);
-    return hipGetLastError();
+    const QueryCopy Q{nq >= kQueryCopyMin ? (Pos3*)c->spos : nullptr, c->max_n, nq};
+    if (Q.spos) {
+        const uint32_t groups = ceil_div(c->max_n, 256u);
+        k_sort_pos<<<groups < 2048u ? groups : 2048u, 256, 0, c->stream>>>(
+            x, y, z, stride, cell_start, g.nx * g.ny * g.nz, sorted_indices, Q);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    constexpr uint32_t kChunk = 1u << 28;  // queries per launch: below 2^32 threads
+    for (uint32_t q0 = 0; q0 < nq; q0 += min(kChunk, nq - q0)) {
+        const uint32_t m = min(kChunk, nq - q0);
+        const size_t o = (size_t)q0 * qstride;
+        k_query<<<ceil_div(m, 256u / kQueryLanes), 256, 0, c->stream>>>(
+            x, y, z, stride, g, cell_start, sorted_indices, qx + o, qy + o, qz + o, qstride, m,
+            radius * radius, counts + q0, offsets ? offsets + q0 : nullptr, indices, Q);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_neighbor_query(fh_ctx* c, const float* x, const float* y, const float* z,

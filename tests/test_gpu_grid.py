@@ -106,6 +106,39 @@ def test_query_batch_matches_oracle(fh, gpu_ctx, oracle):
         assert np.array_equal(got, exp), t
 
 
+@pytest.mark.parametrize("layout", ["aos", "soa"])
+@pytest.mark.parametrize("n,nq", [(1, 1), (40, 1025), (3000, 63), (40_000, 1024), (40_000, 1249),
+                                  (40_000, 1300)])
+def test_query_batch_sizes_match_oracle(fh, gpu_ctx, oracle, layout, n, nq):
+    """Batches on either side of the copy of the positions (1024 queries, a 32nd of the points),
+    rows shorter and longer than a step of 24 candidates, queries outside the grid; a context too
+    small for the grid's points reads them in place."""
+    rng = np.random.default_rng(n + nq)
+    cs, dims = 0.05, (20, 20, 20)
+    p = rng.uniform(0.0, 1.0, (n, 3)).astype(np.float32)
+    p[: n // 2] = 0.4 + 0.1 * p[: n // 2]  # dense: rows of several steps
+    q = rng.uniform(-0.1, 1.1, (nq, 3)).astype(np.float32)
+    q[: nq // 2] = 0.35 + 0.2 * q[: nq // 2]
+    pack = dev if layout == "aos" else lambda a: tuple(dev(a[:, k].copy()) for k in range(3))
+    P, Q = pack(p), pack(q)
+    grid = fh.HashGrid(cs, dims, (0, 0, 0), n, ctx=gpu_ctx)
+    grid.build(P)
+    ocs, osi, _ = oracle.hashgrid_build(p[:, 0], p[:, 1], p[:, 2], cs, (0, 0, 0), dims)
+    small = fh.Context(max_n=16, max_cells=8000)
+    try:
+        for ctx in (gpu_ctx, small):
+            grid.ctx = ctx
+            counts, offsets, idx = (fh.to_u32(t) for t in grid.query_neighbors_batch(Q, 0.04, P))
+            for t in range(0, nq, max(1, nq // 150)):
+                exp = oracle.query_neighbors(q[t], 0.04, p[:, 0], p[:, 1], p[:, 2], cs, (0, 0, 0),
+                                             dims, ocs, osi)
+                assert counts[t] == exp.size
+                assert np.array_equal(idx[offsets[t]:offsets[t + 1]], exp), t
+    finally:
+        grid.ctx = gpu_ctx
+        small.close()
+
+
 @pytest.mark.parametrize("n", [50_000, 4_194_304])
 def test_neighbor_counts_matches_oracle(fh, gpu_ctx, oracle, n):
     """c2 workload (uniform points, r = cs = 0.0122, 82^3 cells); full size at n = 4,194,304."""
