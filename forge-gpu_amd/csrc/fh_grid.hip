@@ -1,12 +1,13 @@
 // fh_grid.hip -- cell ranges and the 3x3x3 neighbour query for gfx950.  (The CSR cell_start
 // of HashGrid::build comes from the sorted keys directly, k_csr_from_sorted in fh_sph.hip.)
 //
-//   k_fill_u32 +   find_cell_boundaries (radix_sort.rs:229-317): sentinel fill, then one
-//   k_boundaries   thread per sorted key marks the first / last index of its run.
+//   k_boundaries   find_cell_boundaries (radix_sort.rs:229-317): one thread per sorted key marks
+//                  the first / last index of its run and the empty cells before it.
 //   k_nbr_stream   HashGrid::query_neighbors (hashgrid.rs:145-193) for every point of a built
 //                  grid: the 3 x-adjacent cells of one (dy, dz) row are contiguous in the
 //                  sorted order, so the 27-cell walk is 9 contiguous ranges visited in the
 //                  reference's dz, dy, dx order.
+#include "fh_cells.hpp"
 #include "fh_internal.hpp"
 #include "fh_stream.hpp"
 
@@ -24,25 +25,50 @@ hipError_t launch_fill_u32(fh_ctx* c, uint32_t* p, uint32_t value, uint32_t n) {
     return hipGetLastError();
 }
 
-// radix_sort.rs:451-465
-__global__ void k_boundaries(const uint32_t* __restrict__ keys, uint32_t n, uint32_t C,
-                             uint32_t* __restrict__ cell_start, uint32_t* __restrict__ cell_end) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t cell = keys[i];
-    if (cell >= C) return;
-    if (i == 0 || keys[i - 1] != cell) cell_start[cell] = i;
-    if (i == n - 1 || keys[i + 1] != cell) cell_end[cell] = i + 1;
+// radix_sort.rs:451-465, in one launch: the slots write the first and the end of their runs and the
+// sentinels of the empty cells before them, and fill_empty_blocks the longer gaps (two fills of
+// every cell and then the runs: 10 us for 300,007 keys of 1,000,000 cells, 7 us this way and two
+// launches fewer).
+__global__ __launch_bounds__(256) void k_boundaries(const uint32_t* __restrict__ keys, uint32_t n,
+                                                    uint32_t C, uint32_t* __restrict__ cell_start,
+                                                    uint32_t* __restrict__ cell_end,
+                                                    uint32_t fill_groups) {
+    const auto empty = [&](uint32_t c, uint32_t) {
+        cell_start[c] = 0xFFFFFFFFu;
+        cell_end[c] = 0u;
+    };
+    if (blockIdx.x < fill_groups) {
+        fill_empty_blocks<false>(blockIdx.x, keys, n, C, empty);
+        return;
+    }
+    const uint32_t s = (blockIdx.x - fill_groups) * 256u + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    uint32_t lo = 0, hi = 0, lo2 = 0, hi2 = 0;
+    if (s < n) {
+        const uint32_t k = keys[s];
+        const uint32_t pk = s > 0u ? keys[s - 1u] : 0xFFFFFFFFu;  // "-1" before slot 0
+        if (s == 0u || pk != k) {
+            lo = min(s == 0u ? 0u : pk + 1u, C);  // pk < k: no wrap
+            hi = min(k, C);
+            if (k < C) cell_start[k] = s;
+        }
+        if (s == n - 1u || keys[s + 1u] != k) {
+            if (k < C) cell_end[k] = s + 1u;
+            if (s == n - 1u) {
+                lo2 = k < C ? k + 1u : C;
+                hi2 = C;
+            }
+        }
+    }
+    fill_cells(lo, hi, C, 0u, lane, empty);
+    if (__ballot(lo2 < hi2) != 0ull) fill_cells(lo2, hi2, C, 0u, lane, empty);
 }
 
 hipError_t launch_boundaries(fh_ctx* c, const uint32_t* sorted_keys, uint32_t n,
                              uint32_t num_cells, uint32_t* cell_start, uint32_t* cell_end) {
-    hipError_t e = launch_fill_u32(c, cell_start, 0xFFFFFFFFu, num_cells);
-    if (e != hipSuccess) return e;
-    e = launch_fill_u32(c, cell_end, 0u, num_cells);
-    if (e != hipSuccess || n == 0) return e;
-    k_boundaries<<<ceil_div(n, 256u), 256, 0, c->stream>>>(sorted_keys, n, num_cells, cell_start,
-                                                           cell_end);
+    const uint32_t fill = empty_block_groups(num_cells);
+    k_boundaries<<<fill + ceil_div(n, 256u), 256, 0, c->stream>>>(sorted_keys, n, num_cells,
+                                                                 cell_start, cell_end, fill);
     return hipGetLastError();
 }
 

@@ -13,6 +13,7 @@
 // visited in the reference's order (dz, dy, dx, then ascending particle id within a cell), so
 // density and velocity updates reproduce the CPU restatement of sph_density.rs:409-460 and
 // sph_fused.rs:542-638.
+#include "fh_cells.hpp"
 #include "fh_internal.hpp"
 #include "fh_stream.hpp"
 
@@ -36,78 +37,6 @@ __global__ __launch_bounds__(256) void k_gather(
     spos[r] = make_float4(px[i], py[i], pz[i], __uint_as_float(r));
     if (svel) svel[r] = make_float4(vx[i], vy[i], vz[i], __uint_as_float(i));
 }
-
-// CSR cell ranges straight from the sorted keys, no scan: the key in slot s starts its run when
-// the key before it, pk, differs; slot s then owns cell_start[c] = s for the cells
-// pk < c <= k (the empty cells before its own take its index: the first sorted index with key
-// >= c), and the last slot also owns the cells after its key up to and including C, which take
-// n.  These ranges partition 0..C, so every entry is written once; together they are the prefix
-// sum of the per-cell counts of hashgrid.rs:102-106.
-//
-// A slot's wave writes its ranges except the blocks of kCellBlock cells (aligned, the last one
-// ending at C) that lie wholly inside one range: those are empty cells between two runs, and the
-// lanes of fill_empty_blocks write them.  Left to the slot, a long gap is one wave's
-// serial store loop: a dam-break block of 1,048,576 particles in the lower part of 100^3 cells
-// leaves ~680,000 cells behind its last key, and k_gather_resident took 312 us with them against
-// 14 us now (k_cell_starts 304 -> 6 us).  What a slot keeps of a gap
-// is at most two partial blocks.
-constexpr uint32_t kCellBlock = 256;
-
-// cell_start[lo..hi) = val without the whole blocks inside (C1 = C + 1 entries in all).  Short
-// ranges are written by their lane, longer ones by the whole wave.
-__device__ __forceinline__ void fill_range(uint32_t* __restrict__ cell_start, uint32_t lo,
-                                           uint32_t hi, uint32_t val, int lane) {
-    const bool mine = hi - lo <= 8u;
-    if (mine)
-        for (uint32_t c = lo; c < hi; c++) cell_start[c] = val;
-    uint64_t wide = __ballot(!mine);
-    while (wide) {  // uniform
-        const int l = __ffsll((unsigned long long)wide) - 1;
-        wide &= wide - 1ull;
-        const uint32_t wlo = (uint32_t)__shfl((int)lo, l, kWave);
-        const uint32_t whi = (uint32_t)__shfl((int)hi, l, kWave);
-        const uint32_t wv = (uint32_t)__shfl((int)val, l, kWave);
-        for (uint32_t c = wlo + (uint32_t)lane; c < whi; c += kWave) cell_start[c] = wv;
-    }
-}
-__device__ __forceinline__ void fill_cells(uint32_t* __restrict__ cell_start, uint32_t lo,
-                                           uint32_t hi, uint32_t C1, uint32_t val, int lane) {
-    const uint32_t first = (lo + kCellBlock - 1u) & ~(kCellBlock - 1u);  // may wrap past 2^32
-    const uint32_t end = hi == C1 ? hi : hi & ~(kCellBlock - 1u);
-    const bool cut = first >= lo && first < end;  // whole blocks [first, end) are not ours
-    fill_range(cell_start, lo, cut ? first : hi, val, lane);
-    if (__ballot(cut && end < hi) != 0ull)
-        fill_range(cell_start, cut ? end : hi, hi, val, lane);
-}
-
-// Blocks of kCellBlock cells, 16 lanes each: a block is written when no key falls in it before
-// its last cell, i.e. when it lies inside one slot's range (the rule fill_cells skips by).  The
-// first slot whose key is >= the block's first cell is searched with 16 probes per round: six
-// dependent rounds for 4,194,304 keys, a third of the loads that 64 probes take in four.  These
-// workgroups come first in the launch, so that the rounds overlap the slots' work (a grid with no
-// long gap pays 0.8 us: 551,368 cells of 4,194,304 uniform points, k_csr_from_sorted 8.7 -> 9.5).
-constexpr uint32_t kBlockLanes = 16, kGroupBlocks16 = 256 / kBlockLanes;
-__device__ __forceinline__ void fill_empty_blocks(uint32_t group, const uint32_t* __restrict__ keys,
-                                                  uint32_t n, uint32_t C,
-                                                  uint32_t* __restrict__ cell_start) {
-    const uint32_t b = group * kGroupBlocks16 + threadIdx.x / kBlockLanes;
-    const uint32_t t = threadIdx.x % kBlockLanes, shift = (threadIdx.x & 63u) & ~(kBlockLanes - 1u);
-    const bool live = b <= C / kCellBlock;
-    const uint32_t c0 = live ? b * kCellBlock : 0u, last = min(c0 + (kCellBlock - 1u), C);
-    uint32_t lo = 0, hi = live ? n : 0u;
-    while (__ballot(lo < hi) != 0ull) {  // until every block of the wave has its slot
-        const uint32_t step = (hi - lo + kBlockLanes - 1u) / kBlockLanes;
-        const uint32_t i = lo + t * step;
-        const bool less = i < hi && keys[min(i, n - 1u)] < c0;
-        const uint32_t below =
-            (uint32_t)__popcll((__ballot(less) >> shift) & ((1ull << kBlockLanes) - 1ull));
-        hi = below ? min(hi, lo + below * step) : lo;
-        lo += below ? (below - 1u) * step + 1u : 0u;
-    }
-    if (!live || (lo < n && keys[lo] < last)) return;
-    for (uint32_t c = t; c <= last - c0; c += kBlockLanes) cell_start[c0 + c] = lo;
-}
-static uint32_t empty_block_groups(uint32_t C) { return C / (kGroupBlocks16 * kCellBlock) + 1u; }
 
 // Cell ranges, and (big != null) the candidate co-located groups: runs of at least
 // kCollapseMin keys in which at least kGroupHits of kGroupSamples evenly spaced particles (over
@@ -138,8 +67,9 @@ __device__ __forceinline__ void cell_starts_slot(uint32_t s, const uint32_t* __r
             hi2 = C + 1u;
         }
     }
-    fill_cells(cell_start, lo, hi, C + 1u, s, lane);
-    if (__ballot(lo2 < hi2) != 0ull) fill_cells(cell_start, lo2, hi2, C + 1u, n, lane);
+    const auto put = [&](uint32_t c, uint32_t v) { cell_start[c] = v; };
+    fill_cells(lo, hi, C + 1u, s, lane, put);
+    if (__ballot(lo2 < hi2) != 0ull) fill_cells(lo2, hi2, C + 1u, n, lane, put);
     // Rare: a run of at least kCollapseMin.  The whole wave takes each such run of its lanes in
     // turn: lane q < kGroupSamples loads sample q (one round trip for all 16); the middle sample
     // is tried first as the group's position, then each other in turn (a corner group can fill
@@ -202,7 +132,8 @@ __global__ __launch_bounds__(256) void k_cell_starts(const uint32_t* __restrict_
                                                      uint64_t* __restrict__ cand_tag,
                                                      Control* ctl, uint32_t fill_groups) {
     if (blockIdx.x < fill_groups) {
-        fill_empty_blocks(blockIdx.x, skeys, n, C, cell_start);
+        fill_empty_blocks<true>(blockIdx.x, skeys, n, C + 1u,
+                                [&](uint32_t c, uint32_t v) { cell_start[c] = v; });
         return;
     }
     cell_starts_slot((blockIdx.x - fill_groups) * blockDim.x + threadIdx.x, skeys, n, C, cell_start,
@@ -210,7 +141,7 @@ __global__ __launch_bounds__(256) void k_cell_starts(const uint32_t* __restrict_
 }
 
 static hipError_t launch_cell_starts(fh_ctx* c, uint32_t cells, uint32_t n, bool list_big) {
-    const uint32_t fill = empty_block_groups(cells);
+    const uint32_t fill = empty_block_groups(cells + 1u);
     tbeg(c, KID_SCAN);
     k_cell_starts<<<fill + ceil_div(n, 256u), 256, 0, c->stream>>>(
         c->skeys, n, cells, c->cell_start, c->spos, list_big ? c->big : nullptr,
@@ -242,7 +173,8 @@ __global__ __launch_bounds__(256) void k_gather_resident(
     uint32_t C, uint32_t* __restrict__ cell_start, uint2* __restrict__ big, uint32_t cap,
     uint64_t* __restrict__ cand_tag, Control* ctl, uint32_t fill_groups) {
     if (blockIdx.x < fill_groups) {
-        fill_empty_blocks(blockIdx.x, skeys, n, C, cell_start);
+        fill_empty_blocks<true>(blockIdx.x, skeys, n, C + 1u,
+                                [&](uint32_t c, uint32_t v) { cell_start[c] = v; });
         return;
     }
     const uint32_t r = (blockIdx.x - fill_groups) * blockDim.x + threadIdx.x;
@@ -260,7 +192,7 @@ __global__ __launch_bounds__(256) void k_gather_resident(
 
 hipError_t launch_gather_resident(fh_ctx* c, uint32_t cells, uint32_t n) {
     if (n == 0) return launch_fill_u32(c, c->cell_start, 0u, cells + 1u);
-    const uint32_t fill = empty_block_groups(cells);
+    const uint32_t fill = empty_block_groups(cells + 1u);
     tbeg(c, KID_GATHER);
     k_gather_resident<<<fill + ceil_div(n, 256u), 256, 0, c->stream>>>(
         c->sout, c->sidx2, n, c->spos, c->svel, c->skeys, cells, c->cell_start, c->big,
@@ -279,7 +211,8 @@ __global__ __launch_bounds__(256) void k_csr_from_sorted(const uint32_t* __restr
                                                          uint32_t* __restrict__ cell_start,
                                                          uint32_t fill_groups) {
     if (blockIdx.x < fill_groups) {
-        fill_empty_blocks(blockIdx.x, keys, n, C, cell_start);
+        fill_empty_blocks<true>(blockIdx.x, keys, n, C + 1u,
+                                [&](uint32_t c, uint32_t v) { cell_start[c] = v; });
         return;
     }
     const uint32_t s = (blockIdx.x - fill_groups) * blockDim.x + threadIdx.x;
@@ -295,14 +228,15 @@ __global__ __launch_bounds__(256) void k_csr_from_sorted(const uint32_t* __restr
             hi2 = C + 1u;
         }
     }
-    fill_cells(cell_start, lo, hi, C + 1u, s, lane);
-    if (__ballot(lo2 < hi2) != 0ull) fill_cells(cell_start, lo2, hi2, C + 1u, n, lane);
+    const auto put = [&](uint32_t c, uint32_t v) { cell_start[c] = v; };
+    fill_cells(lo, hi, C + 1u, s, lane, put);
+    if (__ballot(lo2 < hi2) != 0ull) fill_cells(lo2, hi2, C + 1u, n, lane, put);
 }
 
 hipError_t launch_csr_from_sorted(fh_ctx* c, const uint32_t* keys, uint32_t n, uint32_t cells,
                                   uint32_t* cell_start) {
     if (n == 0) return launch_fill_u32(c, cell_start, 0u, cells + 1u);
-    const uint32_t fill = empty_block_groups(cells);
+    const uint32_t fill = empty_block_groups(cells + 1u);
     k_csr_from_sorted<<<fill + ceil_div(n, 256u), 256, 0, c->stream>>>(
         keys, n, cells, cell_start, fill);
     return hipGetLastError();

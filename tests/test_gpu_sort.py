@@ -207,3 +207,20 @@ def test_find_cell_boundaries_vs_oracle(fh, gpu_ctx, oracle):
     fh.find_cell_boundaries(ids, s, e, keys.size, C, ctx=gpu_ctx)
     os_, oe = oracle.find_cell_boundaries(keys, C)
     assert np.array_equal(fh.to_u32(s), os_) and np.array_equal(fh.to_u32(e), oe)
+
+
+@pytest.mark.parametrize("C", [1, 255, 256, 257, 512, 1000, 100_000])
+@pytest.mark.parametrize("runs", [0, 1, 2, 7, 300])
+def test_find_cell_boundaries_long_gaps(fh, gpu_ctx, oracle, C, runs):
+    """Empty stretches before, between and behind the runs, keys at and beside the edges of the
+    256-cell blocks that are written apart from the slots, keys beyond the grid, no key at all."""
+    rng = np.random.default_rng(1000 * runs + C)
+    edges = np.array([0, 1, 254, 255, 256, 257, 511, 512, 513, C - 1, C, C + 5, 0xFFFFFFFF])
+    picks = np.concatenate([rng.choice(edges, (runs + 1) // 2), rng.integers(0, C + 2, runs // 2)])
+    keys = np.sort(np.repeat(np.maximum(picks, 0), rng.integers(1, 200, runs))).astype(np.uint32)
+    s, e = (torch.full((C,), -7, dtype=torch.int32, device="cuda") for _ in range(2))
+    ids = fh.from_u32(keys)
+    torch.cuda.synchronize()
+    fh.find_cell_boundaries(ids, s, e, keys.size, C, ctx=gpu_ctx)
+    os_, oe = oracle.find_cell_boundaries(keys, C)
+    assert np.array_equal(fh.to_u32(s), os_) and np.array_equal(fh.to_u32(e), oe)
