@@ -275,7 +275,13 @@ int fh_create(int device, uint32_t max_n, uint32_t max_cells, void* stream, fh_c
     if (e == hipSuccess) e = alloc(&c->rank, max_n, &tot);
     if (e == hipSuccess) e = alloc(&c->sout, 3 * (size_t)max_n, &tot);
     if (e == hipSuccess) e = alloc(&c->sidx2, max_n, &tot);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_error, sizeof(uint32_t), hipHostMallocDefault);
+    if (e == hipSuccess)
+        e = hipHostMalloc((void**)&c->h_error, 2 * sizeof(uint32_t), hipHostMallocCoherent);
+    uint32_t* d_error = nullptr;
+    if (e == hipSuccess) {
+        c->h_error[0] = c->h_error[1] = 0u;
+        e = hipHostGetDevicePointer((void**)&d_error, c->h_error, 0);
+    }
     if (e == hipSuccess) {
         if (stream) {
             c->stream = (hipStream_t)stream;
@@ -288,6 +294,9 @@ int fh_create(int device, uint32_t max_n, uint32_t max_cells, void* stream, fh_c
     // (epoch 0 is never current).
     if (e == hipSuccess) e = hipMemsetAsync(c->sort_lb, 0, (size_t)c->max_sort_tiles * kDigitSlots * 4u, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->ctl, 0, sizeof(Control), c->stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(&c->ctl->host_error, &d_error, sizeof(d_error), hipMemcpyHostToDevice,
+                           c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->run_tag, 0, (size_t)max_cells * 8u, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->cell_grp, 0, (size_t)max_cells * 8u, c->stream);
     if (e == hipSuccess)
@@ -342,13 +351,10 @@ int fh_sync(fh_ctx* c) {
     int rc = check_ctx(c);
     if (rc) return rc;
     if (c->capturing) return fail(FH_ESTATE, "fh_sync: stream is being captured");
-    FH_CHECK_HIP(hipMemcpyAsync(c->h_error, &c->ctl->error.v, sizeof(uint32_t),
-                                hipMemcpyDeviceToHost, c->stream));
     FH_CHECK_HIP(hipStreamSynchronize(c->stream));
-    if (*c->h_error) {
-        uint32_t code = *c->h_error;
-        FH_CHECK_HIP(hipMemsetAsync(&c->ctl->error.v, 0, sizeof(uint32_t), c->stream));
-        FH_CHECK_HIP(hipStreamSynchronize(c->stream));
+    volatile uint32_t* const flag = c->h_error;  // stored to by the device (raise_error)
+    if (const uint32_t code = flag[0]) {
+        flag[0] = 0u;
         return fail(FH_ESTATE, "fh_sync: device reported a look-back failure (code %u)", code);
     }
     return FH_OK;
@@ -388,10 +394,10 @@ int fh_sort_plan(fh_ctx* c, uint32_t* plan) {
     if (rc) return rc;
     if (!plan) return fail(FH_EINVAL, "fh_sort_plan: null output");
     if (c->capturing) return fail(FH_ESTATE, "fh_sort_plan: stream is being captured");
-    FH_CHECK_HIP(hipMemcpyAsync(c->h_error, &c->ctl->plan, sizeof(uint32_t),
+    FH_CHECK_HIP(hipMemcpyAsync(c->h_error + 1, &c->ctl->plan, sizeof(uint32_t),
                                 hipMemcpyDeviceToHost, c->stream));
     FH_CHECK_HIP(hipStreamSynchronize(c->stream));
-    *plan = *c->h_error;
+    *plan = c->h_error[1];
     return FH_OK;
 }
 

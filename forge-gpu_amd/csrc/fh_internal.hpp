@@ -132,7 +132,10 @@ struct Control {
     uint32_t epoch;                     // bumped by k_begin before each sort / scan
     uint32_t plan;                      // bit p: sort pass p runs (written by pass 0)
     uint32_t spin_limit;                // look-back polls before giving up (0: kSpinLimit)
-    uint32_t pad0[29];
+    uint32_t pad0;
+    uint32_t* host_error;               // pinned host word of a context that a failure is stored to,
+                                        // or null: to `error` (the no-alloc sort)
+    uint32_t pad1[26];
     Line error;                         // nonzero: a look-back spin limit was hit
     Line tile_ctr[kMaxPasses];          // dynamic tile ids of the sort passes
     Line scan_ctr;                      // dynamic tile id of the cell scan
@@ -245,7 +248,8 @@ struct fh_ctx {
     uint32_t direct_mode; // FH_OPT_DIRECT_ITEMS: 0 never, 1 automatic (default), 2 always
     uint32_t heavy_parts; // FH_OPT_HEAVY_PARTS (0: kHeavyWaves)
     uint32_t sub_bits;    // FH_OPT_SUBCELL: sub-cell key bits of the fused module's fast rebuilds
-    uint32_t* h_error;   // pinned host word for the device error flag
+    uint32_t* h_error;   // pinned host words: [0] the device error flag (Control::host_error),
+                         // which fh_sync reads without a copy, [1] fh_sort_plan's result
     // Epoch renewal.  Tags compare 30-bit epochs, so a tag left 2^30 - 1 starts ago would match
     // again; the host counts the starts it queues (graph replays included) and, before the
     // count reaches epoch_period, queues k_epoch_reset (tags cleared, epoch back to 0).

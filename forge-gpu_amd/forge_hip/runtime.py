@@ -56,6 +56,7 @@ class Context:
         h = ctypes.c_void_p()
         check(lib.fh_create(int(device), int(max_n), int(max_cells), None, ctypes.byref(h)))
         self._h = h
+        self._torch_stream = None
         self.max_n = int(max_n)
         self.max_cells = int(max_cells)
         self.device = int(device)
@@ -71,7 +72,11 @@ class Context:
         return int(_lib.load().fh_stream(self.handle) or 0)
 
     def torch_stream(self) -> torch.cuda.ExternalStream:
-        return torch.cuda.ExternalStream(self.stream_ptr, device=f"cuda:{self.device}")
+        """The context stream as torch sees it (one wrapper per context: the stream never changes)."""
+        if self._torch_stream is None or self._h is None:
+            self._torch_stream = torch.cuda.ExternalStream(self.stream_ptr,
+                                                           device=f"cuda:{self.device}")
+        return self._torch_stream
 
     @property
     def scratch_bytes(self) -> int:
