@@ -112,7 +112,9 @@ __global__ __launch_bounds__(256) void k_gather_pos(const float4* __restrict__ p
 // consecutive sorted points staged through LDS (the wave candidate stream of fh_stream.hpp, one
 // z-slab at a time, kQueryWin candidates per window: a slab's stream of uniform points, ~240
 // candidates, mostly fits one window, so a lane's rows are rarely cut by a window edge and the
-// row loops, which run as long as their longest lane, run once per slab).  Arithmetic is exactly
+// row loops, which run as long as their longest lane, run once per slab).  A candidate is 12 bytes
+// in LDS (16 put neighbouring cells' lanes on the same banks), and a window 384 of them: the
+// query of 4,194,304 points 429 -> 405 us (256: 425, 320: 413, 448: 438).  Arithmetic is exactly
 // the reference's (the library is built with -ffp-contract=off): diff = p_j - q, dist_sq =
 // (dx*dx + dy*dy) + dz*dz, `<=` against radius*radius, weight coeff*diff*diff*diff summed in
 // visiting order; each lane visits its own candidates in the reference's order (dz, dy, then
@@ -120,16 +122,16 @@ __global__ __launch_bounds__(256) void k_gather_pos(const float4* __restrict__ p
 // Points whose query cell lies outside the grid (the reference does not clamp it) take a
 // per-lane walk around that cell afterwards.
 #ifndef FH_QWIN
-#define FH_QWIN 320
+#define FH_QWIN 384
 #endif
 constexpr int kQueryWin = FH_QWIN;
 
 // One candidate: a candidate beyond the radius adds 0 to the count and +0.0f to the weight sum,
 // which starts at +0 and only grows, so w + 0.0f == w bit for bit and the sum over the
 // candidates is the reference's sum over its neighbours.
-__device__ __forceinline__ void nbr_pair(const float4& p, const float4& q, float radius_sq,
-                                         float coeff, uint32_t& cnt, float& w) {
-    const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+__device__ __forceinline__ void nbr_pair(float px, float py, float pz, const float4& q,
+                                         float radius_sq, float coeff, uint32_t& cnt, float& w) {
+    const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
     const float dist_sq = dx * dx + dy * dy + dz * dz;
     const bool ok = dist_sq <= radius_sq;
     const float diff = radius_sq - dist_sq;
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(kWave) void k_nbr_stream(const float4* __restrict__
                                                       uint32_t* __restrict__ counts,
                                                       float* __restrict__ wsum) {
     constexpr int kLoads = kQueryWin / kWave;
-    __shared__ float4 s_p[kQueryWin];
+    __shared__ float s_p[3 * kQueryWin];  // x, y, z
     const int lane = threadIdx.x;
     // runs of consecutive sub-tiles on one XCD: neighbouring sub-tiles read mostly the same
     // candidate rows, which then stay in that XCD's L2
@@ -196,7 +198,12 @@ __global__ __launch_bounds__(kWave) void k_nbr_stream(const float4* __restrict__
             for (int k = 0; k < kLoads; k++) v[k] = spos[j[k]];
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int k = 0; k < kLoads; k++) s_p[k * kWave + lane] = v[k];
+            for (int k = 0; k < kLoads; k++) {
+                float* const o = s_p + 3 * (k * kWave + lane);
+                o[0] = v[k].x;
+                o[1] = v[k].y;
+                o[2] = v[k].z;
+            }
             __builtin_amdgcn_wave_barrier();
             // the rows in the reference's dy order (walking them longest first would change
             // the order of the weight sum)
@@ -208,18 +215,17 @@ __global__ __launch_bounds__(kWave) void k_nbr_stream(const float4* __restrict__
                 // (the bounds are formed from the count, never before the buffer: an address
                 // below the LDS buffer's start would wrap around in 32-bit LDS addressing)
                 const uint32_t m = je > jb ? je - jb : 0u;
-                const float4* c = s_p + (jb - w0);
-                const float4* const ce = c + m;
-                const float4* const cu = c + (m > 1u ? m - 1u : 0u);
-                if (c < cu) {
-                    do {
-                        const float4 p0 = c[0], p1 = c[1];
-                        nbr_pair(p0, q, radius_sq, coeff, cnt, w);
-                        nbr_pair(p1, q, radius_sq, coeff, cnt, w);
-                        c += 2;
-                    } while (c < cu);
+                const float* c = s_p + 3u * (jb - w0);
+                const float* const ce = c + 3u * m;
+                const float* const cu = c + 3u * (m & ~1u);
+                while (c < cu) {
+                    const float x0 = c[0], y0 = c[1], z0 = c[2];
+                    const float x1 = c[3], y1 = c[4], z1 = c[5];
+                    nbr_pair(x0, y0, z0, q, radius_sq, coeff, cnt, w);
+                    nbr_pair(x1, y1, z1, q, radius_sq, coeff, cnt, w);
+                    c += 6;
                 }
-                if (c < ce) nbr_pair(*c, q, radius_sq, coeff, cnt, w);
+                if (c < ce) nbr_pair(c[0], c[1], c[2], q, radius_sq, coeff, cnt, w);
             }
             __builtin_amdgcn_wave_barrier();
         }
@@ -238,7 +244,10 @@ __global__ __launch_bounds__(kWave) void k_nbr_stream(const float4* __restrict__
                 const uint32_t row = (uint32_t)ny * g.nx + (uint32_t)nz * g.nx * g.ny;
                 const uint32_t jb = cell_start[row + (uint32_t)lx0];
                 const uint32_t je = min(cell_start[row + (uint32_t)lx1 + 1u], n);
-                for (uint32_t j = jb; j < je; j++) nbr_pair(spos[j], q, radius_sq, coeff, cnt, w);
+                for (uint32_t j = jb; j < je; j++) {
+                    const float4 p = spos[j];
+                    nbr_pair(p.x, p.y, p.z, q, radius_sq, coeff, cnt, w);
+                }
             }
         }
     }
