@@ -241,8 +241,9 @@ struct fh_ctx {
     uint32_t* rank;      // [max_n] sorted position of each particle (inverse of sidx)
     uint32_t* sidx2;     // [max_n] resident substeps: previous slot of each new slot
     float4* sout;        // [3 * max_n] new state in sorted order before it is moved to particle
-                         // order: pairs (x, y, z, rho), (vx, vy, vz, particle id), then
-                         // (ax, ay, az, .); the next substep's input in resident substeps
+                         // order: pairs (x, y, z, rho), (vx, vy, vz, particle id), the next
+                         // substep's input in resident substeps; with accelerations, records of
+                         // three, the third (ax, ay, az, .)
     bool sph_exact;      // FH_OPT_SPH_EXACT
     uint32_t heavy_work; // FH_OPT_HEAVY_WORK (0: default)
     uint32_t direct_mode; // FH_OPT_DIRECT_ITEMS: 0 never, 1 automatic (default), 2 always
