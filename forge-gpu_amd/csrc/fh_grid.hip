@@ -81,6 +81,10 @@ __device__ __forceinline__ int32_t rust_as_i32(float f) {
     return (int32_t)f;
 }
 
+struct Pos3 {
+    float x, y, z;
+};
+
 // The point positions in sorted order (float4), so the query walks contiguous memory.  A
 // gather through sorted_indices from the caller's three arrays would read three scattered
 // words per point (a cache line each), and a scatter to the sorted slots (through the inverse
@@ -106,6 +110,20 @@ __global__ __launch_bounds__(256) void k_gather_pos(const float4* __restrict__ p
     const uint32_t i = sidx[s];
     // a grid built over these n points holds a permutation of 0..n-1
     spos[s] = i < n ? packed[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
+// The same straight from the caller's 12-byte records (x, y, z adjacent, stride 3): one scattered
+// record per point as from the packed copy, without the pass that makes it (4,194,304 points: build and
+// query 669 -> 637 us; three separate arrays would cost three lines per point).
+__global__ __launch_bounds__(256) void k_gather_aos(const float* __restrict__ xyz,
+                                                    const uint32_t* __restrict__ sidx, uint32_t n,
+                                                    float4* __restrict__ spos) {
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    const uint32_t i = sidx[s];
+    Pos3 p = {0.0f, 0.0f, 0.0f};
+    if (i < n) p = ((const Pos3*)xyz)[i];
+    spos[s] = make_float4(p.x, p.y, p.z, 0.0f);
 }
 
 // HashGrid::query_neighbors for every point of a built grid, with the neighbour candidates of 64
@@ -273,11 +291,8 @@ __global__ __launch_bounds__(kWave) void k_nbr_stream(const float4* __restrict__
 // extra launch would cost more than it gives.  The points' number is the grid's own
 // (cell_start[C]), read on the device; a grid of more points than the context holds is read in place.
 constexpr uint32_t kQueryLanes = 8, kQueryStep = 2, kQueryCopyMin = 1024, kQueryCopyShare = 32;
-struct Pos3 {  // 12 bytes: a row of the copy is a quarter fewer lines than with float4
-    float x, y, z;
-};
 struct QueryCopy {
-    Pos3* spos;      // null: no copy
+    Pos3* spos;      // null: no copy (12 bytes: a row is a quarter fewer lines than with float4)
     uint32_t max_n;  // its room
     uint32_t nq;     // queries of the whole batch
 };
@@ -409,11 +424,16 @@ hipError_t launch_neighbor_query(fh_ctx* c, const float* x, const float* y, cons
                                  const uint32_t* cell_start, const uint32_t* sorted_indices,
                                  float radius, uint32_t* counts, float* wsum) {
     if (n == 0) return hipSuccess;
-    // c->sout (3 float4 per point) is free between SPH calls: the packed copy goes there
-    k_pack_pos<<<ceil_div(n, 256u), 256, 0, c->stream>>>(x, y, z, stride, n, c->sout);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    k_gather_pos<<<ceil_div(n, 256u), 256, 0, c->stream>>>(c->sout, sorted_indices, n, c->spos);
+    hipError_t e;
+    if (stride == 3u && y == x + 1 && z == x + 2) {
+        k_gather_aos<<<ceil_div(n, 256u), 256, 0, c->stream>>>(x, sorted_indices, n, c->spos);
+    } else {
+        // c->sout (3 float4 per point) is free between SPH calls: the packed copy goes there
+        k_pack_pos<<<ceil_div(n, 256u), 256, 0, c->stream>>>(x, y, z, stride, n, c->sout);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        k_gather_pos<<<ceil_div(n, 256u), 256, 0, c->stream>>>(c->sout, sorted_indices, n, c->spos);
+    }
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     // Same float expressions as sph_density.rs:413-416 with h = radius.

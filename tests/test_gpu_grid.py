@@ -194,3 +194,20 @@ def test_neighbor_counts_edge_cases_match_oracle(fh, gpu_ctx, oracle, case):
     assert np.array_equal(fh.to_u32(cnt), ocnt)
     assert np.array_equal(w.cpu().numpy(), ow)
     print(f"{case}: max count {ocnt.max()}, mean {ocnt.mean():.1f}")
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 30_001])
+def test_neighbor_counts_of_records_match_oracle(fh, gpu_ctx, oracle, n):
+    """Positions as 12-byte records, gathered without a packed copy: bit-exact as from arrays."""
+    rng = np.random.default_rng(n)
+    cs, dims = 0.05, (20, 20, 20)
+    p = rng.uniform(-0.02, 1.02, (n, 3)).astype(np.float32)
+    grid = fh.HashGrid(cs, dims, (0, 0, 0), n, ctx=gpu_ctx)
+    P = dev(p)
+    grid.build(P)
+    cnt, w = grid.neighbor_counts(cs, P)
+    x, y, z = (np.ascontiguousarray(p[:, a]) for a in range(3))
+    ocs, osi, _ = oracle.hashgrid_build(x, y, z, grid.cell_size, (0, 0, 0), dims)
+    ocnt, ow = oracle.neighbor_counts(x, y, z, grid.cell_size, (0, 0, 0), dims, ocs, osi, cs)
+    assert np.array_equal(fh.to_u32(cnt), ocnt)
+    assert np.array_equal(w.cpu().numpy(), ow)
