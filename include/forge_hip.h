@@ -262,7 +262,7 @@ int fh_sph_fused_steps(fh_ctx* ctx, const fh_sph_params* prm, const fh_epilogue*
                        float* accel, uint32_t n, float dt, uint32_t steps);
 
 /* Context options.  FH_OPT_SPH_EXACT = 1 makes fh_sph_density / fh_sph_fused evaluate the
- * reference's float expressions term by term in the reference's neighbour order (one thread per
+ * reference's float expressions term by term in the reference's neighbour order (one lane per
  * particle, no FMA, IEEE division and square root: bit-identical to the CPU restatement, slower);
  * 0 (default) uses the LDS-tiled passes (fused multiply-adds, hardware reciprocal square root,
  * deterministic per-slab partial sums; within rel 1e-4). */
