@@ -606,16 +606,16 @@ __device__ __forceinline__ void get_offsets(const uint32_t* __restrict__ off, ui
 // their particles take the representative's density, and its acceleration up to the viscosity
 // term that depends on the particle's own velocity, in k_finalize).  A (sub-tile, slab) item is
 // heavy when its largest per-particle candidate count (a cell that may hold a group counting
-// once) exceeds heavy_work or when it touches such a cell, and transposed (heavy) when its
-// stream is much longer than that count.
+// once) exceeds heavy_work (SMALL: or kSmallHeavyWork, short items with hit masks excepted) or when
+// it touches such a cell, and transposed (heavy) when its stream is much longer than that count.
+template <bool SMALL>
 __device__ __forceinline__ void plan_work(uint32_t bid, const uint32_t* __restrict__ skeys,
                                           uint32_t n, GridDesc g,
                                           const uint32_t* __restrict__ cstart,
                                           const uint64_t* __restrict__ cand_tag,
                                           uint8_t* __restrict__ flag,
                                           uint32_t* __restrict__ heavy, uint32_t heavy_cap,
-                                          uint32_t heavy_work, uint32_t small_work,
-                                          uint32_t direct_mode,
+                                          uint32_t heavy_work, uint32_t direct_mode,
                                           Control* ctl, uint32_t* __restrict__ lstream,
                                           uint2* __restrict__ lstream_t,
                                           uint32_t* __restrict__ hslot, uint32_t hslot_cap) {
@@ -645,10 +645,16 @@ __device__ __forceinline__ void plan_work(uint32_t bid, const uint32_t* __restri
                 const uint32_t w = wave_max(cand);
                 const bool touches = __ballot(excess > 0u) != 0ull;
                 bool hv = w > heavy_work || touches;  // light items hold no group
+                const bool split = SMALL && __ballot(cand > kSmallHeavyWork) != 0ull;
                 bool trans = direct_mode == 2u;
                 LightStream L;
                 L.T = ~0u;  // no stream built
-                bool hits = false;
+                // hit masks: rows of at most 32 candidates (in at most two windows: at most
+                // kMaskWords words), asked before the stream is built, which needs the registers
+                // (asked afterwards, with the small rule as an argument: 42.3 us instead of 40.6
+                // for 1,048,576 particles burst onto the walls of the box)
+                bool hits = direct_mode == 1u && __ballot(cand >= kHitsMin) != 0ull &&
+                            __ballot(max(max(e[0] - b[0], e[1] - b[1]), e[2] - b[2]) > 32u) == 0ull;
                 if (direct_mode == 1u) {
                     // a light item only when its stream is far longer (pathologically
                     // disjoint ranges: one window would serve one lane at a time); the stream
@@ -658,16 +664,13 @@ __device__ __forceinline__ void plan_work(uint32_t bid, const uint32_t* __restri
                     const uint32_t T = build ? L.T : stream_total(b, e, home_row(ci, g), live, lane);
                     trans = hv ? T > kTransRatio * w + kTransOffset
                                : T > kTransLightRatio * w + kTransLightOffset;
-                    // hit masks: rows of at most 32 candidates in at most two windows are at
-                    // most kMaskWords words
-                    hits = w >= kHitsMin && T <= 2u * kWin &&
-                           __ballot(max(max(e[0] - b[0], e[1] - b[1]), e[2] - b[2]) > 32u) == 0ull;
-                    if (!hv && small_work && w > small_work && !(hits && T <= kSmallHitsT)) {
+                    hits = hits && T <= 2u * kWin;
+                    if (!hv && split && !(hits && T <= kSmallHitsT)) {
                         hv = true;
                         trans = T > kTransRatio * w + kTransOffset;
                     }
-                } else if (small_work && w > small_work) {
-                    hv = true;
+                } else {
+                    hv = hv || split;
                 }
                 hv = hv || trans;
                 const uint32_t item = sub * 3u + (uint32_t)slab;
@@ -729,22 +732,23 @@ __device__ __forceinline__ void plan_work(uint32_t bid, const uint32_t* __restri
 constexpr uint32_t kGroupBlocks = 64;
 // 8 waves per SIMD (64 registers, a few spilled): the plan mostly waits on its cell-range loads
 // and the shuffles of the stream build, so occupancy pays more than the registers.
+template <bool SMALL>
 __global__ __launch_bounds__(kPlanThreads, 8) void k_group_plan(
     const uint2* __restrict__ big, uint32_t cap, uint32_t n, const uint32_t* __restrict__ skeys,
     const uint32_t* __restrict__ cstart, float4* __restrict__ spos, float4* __restrict__ svel,
     uint32_t* __restrict__ sidx, uint32_t* __restrict__ rank, uint32_t* __restrict__ scratch,
     uint64_t* __restrict__ cell_grp, float4* __restrict__ vrep, uint32_t* __restrict__ skip_tag,
     GridDesc g, const uint64_t* __restrict__ cand_tag, uint8_t* __restrict__ flag,
-    uint32_t* __restrict__ heavy, uint32_t heavy_cap, uint32_t heavy_work,
-    uint32_t small_work, uint32_t direct_mode, Control* ctl, uint32_t* __restrict__ lstream, uint2* __restrict__ lstream_t,
+    uint32_t* __restrict__ heavy, uint32_t heavy_cap, uint32_t heavy_work, uint32_t direct_mode,
+    Control* ctl, uint32_t* __restrict__ lstream, uint2* __restrict__ lstream_t,
     uint32_t* __restrict__ hslot, uint32_t hslot_cap) {
     if (blockIdx.x < kGroupBlocks)
         group_work(blockIdx.x, kGroupBlocks, big, cap, n, skeys, cstart, spos, svel, sidx, rank,
                    scratch, cell_grp, vrep, skip_tag, ctl);
     else
-        plan_work(blockIdx.x - kGroupBlocks, skeys, n, g, cstart, cand_tag, flag, heavy,
-                  heavy_cap, heavy_work, small_work, direct_mode, ctl, lstream, lstream_t, hslot,
-                  hslot_cap);
+        plan_work<SMALL>(blockIdx.x - kGroupBlocks, skeys, n, g, cstart, cand_tag, flag, heavy,
+                         heavy_cap, heavy_work, direct_mode, ctl, lstream, lstream_t, hslot,
+                         hslot_cap);
 }
 
 // The heavy work lists of this substep as one sequence: entry q of the concatenation of the
@@ -1312,8 +1316,8 @@ static uint32_t heavy_parts(const fh_ctx* c, uint32_t n) {
 static uint32_t heavy_work(const fh_ctx* c) {
     return c->heavy_work ? c->heavy_work : kHeavyWork;
 }
-static uint32_t small_work(const fh_ctx* c, uint32_t n) {
-    return !c->heavy_work && n < kSmallSystemN ? kSmallHeavyWork : 0u;
+static bool small_rule(const fh_ctx* c, uint32_t n) {
+    return !c->heavy_work && n < kSmallSystemN;
 }
 static uint32_t heavy_grid(uint32_t items) {
     const uint32_t g = (items / 8u + 7u) / 8u * 8u;
@@ -2053,14 +2057,12 @@ hipError_t launch_group_plan(fh_ctx* c, const SphArgs& a, bool with_vel) {
     if (a.n == 0) return hipSuccess;
     // scratch of the group part: the sort's key buffer, free after the sort (disjoint ranges per cell)
     tbeg(c, KID_PLAN);
-    k_group_plan<<<kGroupBlocks + ceil_div(a.n, (uint32_t)kPlanThreads), kPlanThreads, 0,
-                   c->stream>>>(c->big, ceil_div(c->max_n, 64u) + 1u, a.n, c->skeys, c->cell_start,
-                                c->spos, with_vel ? c->svel : nullptr, c->sidx, c->rank, c->ka,
-                                c->cell_grp, c->vrep, c->skip_tag, a.g, c->run_tag,
-                                c->heavy_flag, c->heavy, c->heavy_cap,
-                                heavy_work(c), small_work(c, a.n), c->direct_mode,
-                                c->ctl, c->lstream, c->lstream_t, c->hslot,
-                                slot_cap(c, heavy_parts(c, a.n)));
+    const auto kernel = small_rule(c, a.n) ? k_group_plan<true> : k_group_plan<false>;
+    kernel<<<kGroupBlocks + ceil_div(a.n, (uint32_t)kPlanThreads), kPlanThreads, 0, c->stream>>>(
+        c->big, ceil_div(c->max_n, 64u) + 1u, a.n, c->skeys, c->cell_start, c->spos,
+        with_vel ? c->svel : nullptr, c->sidx, c->rank, c->ka, c->cell_grp, c->vrep, c->skip_tag,
+        a.g, c->run_tag, c->heavy_flag, c->heavy, c->heavy_cap, heavy_work(c), c->direct_mode,
+        c->ctl, c->lstream, c->lstream_t, c->hslot, slot_cap(c, heavy_parts(c, a.n)));
     tend(c, KID_PLAN);
     return hipGetLastError();
 }
