@@ -290,6 +290,8 @@ __global__ __launch_bounds__(kWave) void k_nbr_stream(const float4* __restrict__
 // one query per hundred points: batches of at least a 32nd of the points make it, and below kQueryCopyMin queries the
 // extra launch would cost more than it gives.  The points' number is the grid's own
 // (cell_start[C]), read on the device; a grid of more points than the context holds is read in place.
+// An id of that number or more (a grid over some of an array's points, an entry that no query comes
+// near) is not followed by the copy, which leaves a NaN: its position is read where a query meets it.
 constexpr uint32_t kQueryLanes = 8, kQueryStep = 2, kQueryCopyMin = 1024, kQueryCopyShare = 32;
 struct QueryCopy {
     Pos3* spos;      // null: no copy (12 bytes: a row is a quarter fewer lines than with float4)
@@ -309,8 +311,12 @@ __global__ __launch_bounds__(256) void k_sort_pos(const float* __restrict__ x,
     const uint32_t n = cstart[C];
     if (!query_copied(Q, n)) return;
     for (uint32_t s = blockIdx.x * 256u + threadIdx.x; s < n; s += gridDim.x * 256u) {
-        const size_t o = (size_t)sidx[s] * stride;
-        Q.spos[s] = Pos3{x[o], y[o], z[o]};
+        const uint32_t i = sidx[s];
+        const size_t o = (size_t)(i < n ? i : 0u) * stride;
+        const float nan = __builtin_nanf("");
+        Pos3 p = {x[o], y[o], z[o]};
+        if (i >= n) p = Pos3{nan, nan, nan};
+        Q.spos[s] = p;
     }
 }
 
@@ -349,6 +355,12 @@ __global__ __launch_bounds__(256) void k_query(const float* __restrict__ x,
         e = min(cstart[row + (uint32_t)x1 + 1u], n);
         b = cstart[row + (uint32_t)x0];
     };
+    const auto in_place = [&](uint32_t j, float& X, float& Y, float& Z) {
+        const size_t o = (size_t)sidx[j] * stride;
+        X = x[o];
+        Y = y[o];
+        Z = z[o];
+    };
     uint32_t b0, e0, b8, e8;
     range(t, b0, e0);
     range(8u, b8, e8);
@@ -369,11 +381,14 @@ __global__ __launch_bounds__(256) void k_query(const float* __restrict__ x,
                     Y[k] = p.y;
                     Z[k] = p.z;
                 } else {
-                    const size_t o = (size_t)sidx[j] * stride;
-                    X[k] = x[o];
-                    Y[k] = y[o];
-                    Z[k] = z[o];
+                    in_place(j, X[k], Y[k], Z[k]);
                 }
+            }
+            static_assert(kQueryStep == 2, "one compare asks both candidates of a step");
+            if (copied && __builtin_isunordered(X[0], X[1])) {  // (a NaN point reads the same again)
+#pragma unroll
+                for (uint32_t k = 0; k < kQueryStep; k++)
+                    in_place(min(j0 + k * kQueryLanes + t, e - 1u), X[k], Y[k], Z[k]);
             }
 #pragma unroll
             for (uint32_t k = 0; k < kQueryStep; k++) {

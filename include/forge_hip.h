@@ -186,7 +186,10 @@ int fh_neighbor_query(fh_ctx* ctx, const float* x, const float* y, const float* 
  * cell order) and kept when ((dx*dx + dy*dy) + dz*dz) <= radius^2 with dx = p_j - q.
  * counts[q] receives the number of neighbours.  If `offsets` (nq+1 exclusive prefix sums of a
  * previous count call) and `indices` are non-NULL, the neighbour ids of query q are also
- * written to indices[offsets[q] .. offsets[q+1]). */
+ * written to indices[offsets[q] .. offsets[q+1]).  Batches of 1,024 or more queries may first copy
+ * the grid's positions into the context's scratch, so every id below cell_start[C] among
+ * sorted_indices[0 .. cell_start[C]) must have a position; larger ids (a grid over some of the
+ * points of x/y/z) are followed only where a query comes near them. */
 int fh_query_neighbors(fh_ctx* ctx, const float* x, const float* y, const float* z,
                        uint32_t stride, float cell_size, const float origin[3],
                        const uint32_t dims[3], const uint32_t* cell_start,

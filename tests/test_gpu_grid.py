@@ -139,6 +139,37 @@ def test_query_batch_sizes_match_oracle(fh, gpu_ctx, oracle, layout, n, nq):
         small.close()
 
 
+@pytest.mark.parametrize("kind", ["subset", "far"])
+def test_query_batch_over_part_of_the_points(fh, gpu_ctx, oracle, kind):
+    """A batch that copies the positions reads no more of the caller's arrays than it may: a grid
+    over some of the points (ids beyond the grid's own count), and entries that hold no id at all in
+    cells that no query comes near."""
+    rng = np.random.default_rng(17)
+    cs, dims, total, n = 0.05, (20, 20, 20), 60_000, 40_000
+    p = rng.uniform(0.0, 1.0, (total, 3)).astype(np.float32)
+    ids = np.sort(rng.permutation(total)[:n]) if kind == "subset" else np.arange(n)
+    sub = p[ids]
+    ocs, osi, cell = oracle.hashgrid_build(sub[:, 0], sub[:, 1], sub[:, 2], cs, (0, 0, 0), dims)
+    near = ids[osi].astype(np.uint32)
+    q = rng.uniform(0.0, 1.0, (2000, 3)).astype(np.float32)
+    given = near.copy()
+    if kind == "far":
+        q[:, 0] *= 0.5  # cells x < 10, rows up to x = 10
+        given[cell[osi] % 20 >= 12] = 0xFFFFFFF0
+        p = p[:n]
+    P = tuple(dev(p[:, k].copy()) for k in range(3))
+    grid = fh.HashGrid(cs, dims, (0, 0, 0), n, ctx=gpu_ctx)
+    grid.build(tuple(dev(sub[:, k].copy()) for k in range(3)))
+    grid.sorted_indices[:n] = fh.from_u32(given)
+    torch.cuda.synchronize()
+    counts, offsets, idx = (fh.to_u32(t) for t in grid.query_neighbors_batch(dev(q), 0.04, P))
+    for t in range(0, len(q), 13):
+        exp = oracle.query_neighbors(q[t], 0.04, p[:, 0], p[:, 1], p[:, 2], cs, (0, 0, 0), dims,
+                                     ocs, near)
+        assert counts[t] == exp.size
+        assert np.array_equal(idx[offsets[t]:offsets[t + 1]], exp), t
+
+
 @pytest.mark.parametrize("n", [50_000, 4_194_304])
 def test_neighbor_counts_matches_oracle(fh, gpu_ctx, oracle, n):
     """c2 workload (uniform points, r = cs = 0.0122, 82^3 cells); full size at n = 4,194,304."""
