@@ -22,21 +22,24 @@ namespace fh {
 // 14 us now (k_cell_starts 304 -> 6 us).  What a slot keeps of a gap is at most two partial blocks.
 constexpr uint32_t kCellBlock = 256;
 
-// put(c, val) for the cells [lo, hi): short ranges by their lane, longer ones by the whole wave.
+// put(c, val) for the cells [lo, hi) (none if hi <= lo): short ranges by their lane, longer ones by
+// the whole wave, which steps through offsets: a cell number near 2^32 would wrap around.
 template <class Put>
 __device__ __forceinline__ void fill_range(uint32_t lo, uint32_t hi, uint32_t val, int lane,
                                            Put&& put) {
-    const bool mine = hi - lo <= 8u;
+    const uint32_t len = hi > lo ? hi - lo : 0u;
+    const bool mine = len <= 8u;
     if (mine)
-        for (uint32_t c = lo; c < hi; c++) put(c, val);
+        for (uint32_t o = 0; o < len; o++) put(lo + o, val);
     uint64_t wide = __ballot(!mine);
     while (wide) {  // uniform
         const int l = __ffsll((unsigned long long)wide) - 1;
         wide &= wide - 1ull;
         const uint32_t wlo = (uint32_t)__shfl((int)lo, l, kWave);
-        const uint32_t whi = (uint32_t)__shfl((int)hi, l, kWave);
+        const uint32_t wlen = (uint32_t)__shfl((int)len, l, kWave);
         const uint32_t wv = (uint32_t)__shfl((int)val, l, kWave);
-        for (uint32_t c = wlo + (uint32_t)lane; c < whi; c += kWave) put(c, wv);
+        // (wlen < 2 * kCellBlock: fill_cells leaves the whole blocks out)
+        for (uint32_t o = (uint32_t)lane; o < wlen; o += kWave) put(wlo + o, wv);
     }
 }
 // The same without the whole blocks inside, of `entries` cells in all.

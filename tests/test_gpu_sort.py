@@ -224,3 +224,26 @@ def test_find_cell_boundaries_long_gaps(fh, gpu_ctx, oracle, C, runs):
     fh.find_cell_boundaries(ids, s, e, keys.size, C, ctx=gpu_ctx)
     os_, oe = oracle.find_cell_boundaries(keys, C)
     assert np.array_equal(fh.to_u32(s), os_) and np.array_equal(fh.to_u32(e), oe)
+
+
+def test_cell_ranges_of_the_largest_grids(fh, gpu_ctx):
+    """2^32 - 1 cells (and a CSR of as many entries): empty cells up to the last cell number."""
+    C = 0xFFFFFFFF
+    keys = np.array([0, 255, 255, 0xFFFFFF10, 0xFFFFFF10, 0xFFFFFFE0], np.uint32)
+    ids = fh.from_u32(keys)
+    s, e = (torch.full((C,), -7, dtype=torch.int32, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    fh.find_cell_boundaries(ids, s, e, keys.size, C, ctx=gpu_ctx)
+    cells = torch.from_numpy(np.unique(keys).astype(np.int64)).cuda()
+    assert s[cells].tolist() == [0, 1, 3, 5] and e[cells].tolist() == [1, 3, 5, 6]
+    s[cells] = -1
+    e[cells] = 0
+    assert bool((s == -1).all()) and bool((e == 0).all())
+    del e
+    fh.cell_start_csr(ids, keys.size, C - 1, s, ctx=gpu_ctx)  # s[c]: number of keys below c
+    at = 0
+    for v, k in enumerate(np.append(keys, np.uint32(C - 1))):
+        assert bool((s[at:int(k) + 1] == v).all())
+        at = int(k) + 1
+    del s
+    torch.cuda.empty_cache()
