@@ -87,4 +87,22 @@ inline uint32_t empty_block_groups(uint32_t entries) {
     return (entries - 1u) / (kGroupBlocks16 * kCellBlock) + 1u;
 }
 
+// launch(groups, fill_groups): the blocks of `entries` cells and the slots of n keys in one launch,
+// or, where that would be 2^32 threads or more, in one each (more keys than one launch takes: refused).
+template <class Launch>
+hipError_t launch_cell_groups(uint32_t n, uint32_t entries, Launch&& launch) {
+    constexpr uint32_t kMaxGroups = (1u << 24) - 1u;
+    const uint32_t fill = empty_block_groups(entries), slots = n / 256u + (n % 256u != 0u);
+    if (slots > kMaxGroups) return hipErrorInvalidConfiguration;
+    if (fill + slots <= kMaxGroups) {
+        launch(fill + slots, fill);
+        return hipGetLastError();
+    }
+    launch(fill, fill);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    launch(slots, 0u);
+    return hipGetLastError();
+}
+
 }  // namespace fh

@@ -66,10 +66,10 @@ __global__ __launch_bounds__(256) void k_boundaries(const uint32_t* __restrict__
 
 hipError_t launch_boundaries(fh_ctx* c, const uint32_t* sorted_keys, uint32_t n,
                              uint32_t num_cells, uint32_t* cell_start, uint32_t* cell_end) {
-    const uint32_t fill = empty_block_groups(num_cells);
-    k_boundaries<<<fill + ceil_div(n, 256u), 256, 0, c->stream>>>(sorted_keys, n, num_cells,
-                                                                 cell_start, cell_end, fill);
-    return hipGetLastError();
+    return launch_cell_groups(n, num_cells, [&](uint32_t groups, uint32_t fill) {
+        k_boundaries<<<groups, 256, 0, c->stream>>>(sorted_keys, n, num_cells, cell_start, cell_end,
+                                                    fill);
+    });
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -236,10 +236,9 @@ __global__ __launch_bounds__(256) void k_csr_from_sorted(const uint32_t* __restr
 hipError_t launch_csr_from_sorted(fh_ctx* c, const uint32_t* keys, uint32_t n, uint32_t cells,
                                   uint32_t* cell_start) {
     if (n == 0) return launch_fill_u32(c, cell_start, 0u, cells + 1u);
-    const uint32_t fill = empty_block_groups(cells + 1u);
-    k_csr_from_sorted<<<fill + ceil_div(n, 256u), 256, 0, c->stream>>>(
-        keys, n, cells, cell_start, fill);
-    return hipGetLastError();
+    return launch_cell_groups(n, cells + 1u, [&](uint32_t groups, uint32_t fill) {
+        k_csr_from_sorted<<<groups, 256, 0, c->stream>>>(keys, n, cells, cell_start, fill);
+    });
 }
 
 // Sorted-order state for the exact passes over a caller's grid (sorted_indices[s] = the particle in

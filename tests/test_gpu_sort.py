@@ -247,3 +247,27 @@ def test_cell_ranges_of_the_largest_grids(fh, gpu_ctx):
         at = int(k) + 1
     del s
     torch.cuda.empty_cache()
+
+
+def test_cell_ranges_of_the_most_keys(fh, gpu_ctx):
+    """As many keys as one launch takes a thread each for, so that the empty cells are a launch of
+    their own; more keys are refused."""
+    n, C = (1 << 32) - 512, 5000
+    ids = torch.zeros(n, dtype=torch.int32, device="cuda")
+    ids[-3:] = torch.tensor([300, 4500, 4500], dtype=torch.int32, device="cuda")
+    s, e = (torch.full((C,), -7, dtype=torch.int32, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    fh.find_cell_boundaries(ids, s, e, n, C, ctx=gpu_ctx)
+    start, end = np.full(C, 0xFFFFFFFF, np.uint32), np.zeros(C, np.uint32)
+    start[[0, 300, 4500]], end[[0, 300, 4500]] = [0, n - 3, n - 2], [n - 3, n - 2, n]
+    assert np.array_equal(fh.to_u32(s), start) and np.array_equal(fh.to_u32(e), end)
+    csr = torch.full((C + 1,), -7, dtype=torch.int32, device="cuda")
+    fh.cell_start_csr(ids, n, C, csr, ctx=gpu_ctx)
+    below = np.repeat(np.array([0, n - 3, n - 2, n], np.uint32), [1, 300, 4200, 500])
+    assert np.array_equal(fh.to_u32(csr), below)
+    for call in (lambda: fh.find_cell_boundaries(ids, s, e, n + 257, C, ctx=gpu_ctx),
+                 lambda: fh.cell_start_csr(ids, n + 257, C, csr, ctx=gpu_ctx)):
+        with pytest.raises(fh.ForgeError):
+            call()
+    del ids
+    torch.cuda.empty_cache()
