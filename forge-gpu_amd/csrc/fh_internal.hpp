@@ -195,11 +195,10 @@ struct fh_ctx {
     uint32_t max_n, max_cells;
     uint32_t max_sort_tiles;
     // sort scratch
-    uint32_t* ka;        // [max_n], then va and vb sort_stride words apart in the same allocation
-    uint32_t* va;        // [max_n] (a HitPlanes plane between the density and the force pass)
-    uint32_t* vb;        // [max_n]
-    uint32_t sort_stride; // max_n rounded up to whole 256-byte rows of a wave
+    uint32_t* ka;        // [max_n] (ka, va, vb: HitPlanes planes between the density and the force
+    uint32_t* va;        // [max_n]  pass)
     uint32_t* kb;        // [max_n]
+    uint32_t* vb;        // [max_n]
     uint32_t* sort_lb;   // [max_sort_tiles * kDigitSlots] 32-bit look-back words (pass-major)
     uint32_t* hist_part; // [kHistBlocks][kDigitSlots] per-block digit histograms
     uint32_t* sort_pre;  // first-pass tile prefixes of small sorts (tiles of pre_rows_per_tile

@@ -916,14 +916,16 @@ __device__ __forceinline__ uint32_t density_hits(const float* __restrict__ p, ui
 // acceleration partials (by the wave that has read the masks), word 3 in the sort's ping-pong
 // buffers, word 4 in the last third of sout (written by k_finalize), word 5 in hits.
 struct HitPlanes {
-    uint32_t* f;             // fpart
-    uint32_t *w3, *w4, *w5;  // [3][stride3], then [3][stride] each
-    uint32_t stride, stride3;
+    uint32_t* f;                // fpart
+    uint32_t *w3a, *w3b, *w3c;  // a slab each, [stride]
+    uint32_t *w4, *w5;          // [3][stride] each
+    uint32_t stride;
 };
 __device__ __forceinline__ uint32_t* hit_word(const HitPlanes& H, uint32_t slab, uint32_t q) {
     // (selects: an indexed member would put the argument into scratch memory)
-    uint32_t* const p = q < 3u ? H.f : (q == 3u ? H.w3 : (q == 4u ? H.w4 : H.w5));
-    return p + (size_t)(q < 3u ? slab * 3u + q : slab) * (q == 3u ? H.stride3 : H.stride);
+    if (q == 3u) return slab == 0u ? H.w3a : (slab == 1u ? H.w3b : H.w3c);
+    uint32_t* const p = q < 3u ? H.f : (q == 4u ? H.w4 : H.w5);
+    return p + (size_t)(q < 3u ? slab * 3u + q : slab) * H.stride;
 }
 
 // Density partials: dpart[slab][s] = sum over the slab's neighbours j of (h^2 - r^2)^3, r^2 < h^2.
@@ -2068,8 +2070,8 @@ hipError_t launch_group_plan(fh_ctx* c, const SphArgs& a, bool with_vel) {
 }
 
 static HitPlanes hit_planes(fh_ctx* c) {
-    return HitPlanes{(uint32_t*)c->fpart, c->ka, (uint32_t*)(c->sout + 2 * (size_t)c->max_n),
-                     c->hits, c->max_n, c->sort_stride};
+    return HitPlanes{(uint32_t*)c->fpart, c->ka, c->va, c->vb,
+                     (uint32_t*)(c->sout + 2 * (size_t)c->max_n), c->hits, c->max_n};
 }
 
 hipError_t launch_density_fast(fh_ctx* c, const SphArgs& a, const uint32_t* cell_start,
