@@ -284,31 +284,46 @@ __global__ __launch_bounds__(kWave) void k_nbr_stream(const float4* __restrict__
 // Positions come from a copy in slot order when the batch is large (k_sort_pos), where a row is a few
 // contiguous lines; read through sorted_indices from the caller's arrays every candidate is a line
 // (two more in three separate arrays), and a lane per query waits for them one after the other.
-// 120,000 queries in 600,000 points: 333 us for a count or fill pass with a lane per query, 83 us
-// with eight, the copy (11 us) included; 4, 16 and 32 lanes 110, 82 and 80, and 94 with 16-byte
-// positions: the rows' lines, which mostly miss a 4 MB L2, are what is left.  The copy pays from about
-// one query per hundred points: batches of at least a 32nd of the points make it, and below kQueryCopyMin queries the
-// extra launch would cost more than it gives.  The points' number is the grid's own
+// 120,000 queries in 600,000 points: 333 us for a count or fill pass with a lane per query, 67 us
+// with eight, the copy (11 us) included (83 while both ways to the positions shared a loop); 4, 16 and
+// 32 lanes 110, 82 and 80 against those 83, and 94 with 16-byte positions: the rows' lines, which
+// mostly miss a 4 MB L2, are what is left.
+//
+// The copy reads every point once, so it pays from a number of candidates per point on: 2.5, or, where
+// the caller's positions themselves stay in the L2, 12.  2,000,000 points, 200,000 queries: 4
+// neighbours each (2.6 candidates per point) 106 us against 145 in place; 2 (1.3) 114 against 104; 0.5
+// (0.3) 95 against 64.  600,000 points, 30 neighbours: 7,000 queries (2.3) 38 against 34.  100,000
+// points and queries: 3 neighbours (19) 30 against 33, 1 (6.4) 28 against 24.  Below kQueryCopyMin
+// queries the extra launch would cost more than it gives.  The points' number is the grid's own
 // (cell_start[C]), read on the device; a grid of more points than the context holds is read in place.
 // An id of that number or more (a grid over some of an array's points, an entry that no query comes
 // near) is not followed by the copy, which leaves a NaN: its position is read where a query meets it.
-constexpr uint32_t kQueryLanes = 8, kQueryStep = 2, kQueryCopyMin = 1024, kQueryCopyShare = 32;
+constexpr uint32_t kQueryLanes = 8, kQueryStep = 2, kQueryCopyMin = 1024;
+constexpr uint32_t kQueryCopyShare = 5, kQueryCacheShare = 24, kQueryCacheN = 1u << 18;
 struct QueryCopy {
     Pos3* spos;      // null: no copy (12 bytes: a row is a quarter fewer lines than with float4)
     uint32_t max_n;  // its room
     uint32_t nq;     // queries of the whole batch
+    uint32_t C;      // cells
 };
+// Whether the batch meets at least `share` / 2 candidates per point of the grid: 27 n / C per query.
+__host__ __device__ __forceinline__ bool query_candidates(uint32_t nq, uint32_t C, uint32_t share) {
+    return (uint64_t)nq * 54u >= (uint64_t)C * share;
+}
+__host__ __device__ __forceinline__ uint32_t query_share(uint32_t n) {
+    return n < kQueryCacheN ? kQueryCacheShare : kQueryCopyShare;
+}
 __device__ __forceinline__ bool query_copied(const QueryCopy& Q, uint32_t n) {
-    return Q.spos && n <= Q.max_n && (uint64_t)Q.nq * kQueryCopyShare >= n;
+    return Q.spos && n <= Q.max_n && query_candidates(Q.nq, Q.C, query_share(n));
 }
 
 __global__ __launch_bounds__(256) void k_sort_pos(const float* __restrict__ x,
                                                   const float* __restrict__ y,
                                                   const float* __restrict__ z, uint32_t stride,
-                                                  const uint32_t* __restrict__ cstart, uint32_t C,
+                                                  const uint32_t* __restrict__ cstart,
                                                   const uint32_t* __restrict__ sidx,
                                                   QueryCopy Q) {
-    const uint32_t n = cstart[C];
+    const uint32_t n = cstart[Q.C];
     if (!query_copied(Q, n)) return;
     for (uint32_t s = blockIdx.x * 256u + threadIdx.x; s < n; s += gridDim.x * 256u) {
         const uint32_t i = sidx[s];
@@ -336,7 +351,7 @@ __global__ __launch_bounds__(256) void k_query(const float* __restrict__ x,
     const uint32_t shift = (threadIdx.x & 63u) & ~(kQueryLanes - 1u);
     const uint32_t qi = (blockIdx.x * 256u + threadIdx.x) / kQueryLanes;
     if (qi >= nq) return;  // whole groups
-    const uint32_t n = cstart[g.nx * g.ny * g.nz];
+    const uint32_t n = cstart[Q.C];
     const bool copied = query_copied(Q, n);  // uniform
     const size_t oq = (size_t)qi * qstride;
     const float px = qx[oq], py = qy[oq], pz = qz[oq];
@@ -355,40 +370,41 @@ __global__ __launch_bounds__(256) void k_query(const float* __restrict__ x,
         e = min(cstart[row + (uint32_t)x1 + 1u], n);
         b = cstart[row + (uint32_t)x0];
     };
-    const auto in_place = [&](uint32_t j, float& X, float& Y, float& Z) {
-        const size_t o = (size_t)sidx[j] * stride;
-        X = x[o];
-        Y = y[o];
-        Z = z[o];
-    };
     uint32_t b0, e0, b8, e8;
     range(t, b0, e0);
     range(8u, b8, e8);
     uint32_t cnt = 0;
     uint32_t* out = (offsets && indices) ? indices + offsets[qi] : nullptr;
     const uint32_t room = out ? offsets[qi + 1] - offsets[qi] : 0u;
-    for (uint32_t r = 0; r < 9u; r++) {
+    const auto row = [&](uint32_t r) {
         const uint32_t b = r < 8u ? (uint32_t)__shfl((int)b0, (int)r, (int)kQueryLanes) : b8;
         const uint32_t e = r < 8u ? (uint32_t)__shfl((int)e0, (int)r, (int)kQueryLanes) : e8;
         for (uint32_t j0 = b; j0 < e; j0 += kQueryStep * kQueryLanes) {  // uniform in the group
             float X[kQueryStep], Y[kQueryStep], Z[kQueryStep];
+            bool read = !copied;
+            if (copied) {
 #pragma unroll
-            for (uint32_t k = 0; k < kQueryStep; k++) {
-                const uint32_t j = min(j0 + k * kQueryLanes + t, e - 1u);
-                if (copied) {
-                    const Pos3 p = Q.spos[j];
+                for (uint32_t k = 0; k < kQueryStep; k++) {
+                    const Pos3 p = Q.spos[min(j0 + k * kQueryLanes + t, e - 1u)];
                     X[k] = p.x;
                     Y[k] = p.y;
                     Z[k] = p.z;
-                } else {
-                    in_place(j, X[k], Y[k], Z[k]);
                 }
+                static_assert(kQueryStep == 2, "one compare asks both candidates of a step");
+                read = __builtin_isunordered(X[0], X[1]);  // (a point that is NaN reads the same again)
             }
-            static_assert(kQueryStep == 2, "one compare asks both candidates of a step");
-            if (copied && __builtin_isunordered(X[0], X[1])) {  // (a NaN point reads the same again)
+            if (read) {
+                uint32_t i[kQueryStep];
 #pragma unroll
                 for (uint32_t k = 0; k < kQueryStep; k++)
-                    in_place(min(j0 + k * kQueryLanes + t, e - 1u), X[k], Y[k], Z[k]);
+                    i[k] = sidx[min(j0 + k * kQueryLanes + t, e - 1u)];
+#pragma unroll
+                for (uint32_t k = 0; k < kQueryStep; k++) {
+                    const size_t o = (size_t)i[k] * stride;
+                    X[k] = x[o];
+                    Y[k] = y[o];
+                    Z[k] = z[o];
+                }
             }
 #pragma unroll
             for (uint32_t k = 0; k < kQueryStep; k++) {
@@ -403,6 +419,16 @@ __global__ __launch_bounds__(256) void k_query(const float* __restrict__ x,
                 cnt += (uint32_t)__popc(m);
             }
         }
+    };
+    // the rows in order: all nine, or, where more than three in eight of the wave's are empty, those
+    // that hold points (uniform in the group; 100,000 queries of 0.3 neighbours 30 -> 21 us)
+    const uint64_t held = __ballot(b0 < e0);
+    if (__popcll(held) >= 40) {
+        for (uint32_t r = 0; r < 9u; r++) row(r);
+    } else {
+        uint32_t rows = (uint32_t)(held >> shift) & ((1u << kQueryLanes) - 1u);
+        rows |= b8 < e8 ? 1u << 8 : 0u;
+        for (; rows; rows &= rows - 1u) row((uint32_t)__builtin_ctz(rows));
     }
     if (t == 0u) counts[qi] = cnt;
 }
@@ -413,11 +439,13 @@ hipError_t launch_query(fh_ctx* c, const float* x, const float* y, const float* 
                         const float* qz, uint32_t qstride, uint32_t nq, float radius,
                         uint32_t* counts, const uint32_t* offsets, uint32_t* indices) {
     if (nq == 0) return hipSuccess;
-    const QueryCopy Q{nq >= kQueryCopyMin ? (Pos3*)c->spos : nullptr, c->max_n, nq};
+    const uint32_t C = g.nx * g.ny * g.nz;
+    const bool copy = nq >= kQueryCopyMin && query_candidates(nq, C, query_share(c->max_n));
+    const QueryCopy Q{copy ? (Pos3*)c->spos : nullptr, c->max_n, nq, C};
     if (Q.spos) {
         const uint32_t groups = ceil_div(c->max_n, 256u);
         k_sort_pos<<<groups < 2048u ? groups : 2048u, 256, 0, c->stream>>>(
-            x, y, z, stride, cell_start, g.nx * g.ny * g.nz, sorted_indices, Q);
+            x, y, z, stride, cell_start, sorted_indices, Q);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -139,6 +139,28 @@ def test_query_batch_sizes_match_oracle(fh, gpu_ctx, oracle, layout, n, nq):
         small.close()
 
 
+@pytest.mark.parametrize("n,nq", [(300, 3555), (300, 3556), (6000, 1100), (6000, 3555),
+                                  (30_000, 3556), (262_143, 3555), (262_143, 3556),
+                                  (262_144, 1024)])
+def test_query_batch_rules_match_oracle(fh, gpu_ctx, oracle, n, nq):
+    """On either side of the copy's rule (12 candidates per point, 2.5 from 2^18 points on) and of the
+    walk over rows that hold points only: few points per row, empty rows, full ones."""
+    rng = np.random.default_rng(n + nq)
+    cs, dims = 0.05, (20, 20, 20)
+    p = rng.uniform(0.0, 1.0, (n, 3)).astype(np.float32)
+    q = rng.uniform(-0.05, 1.05, (nq, 3)).astype(np.float32)
+    grid = fh.HashGrid(cs, dims, (0, 0, 0), n, ctx=gpu_ctx)
+    P = dev(p)
+    grid.build(P)
+    ocs, osi, _ = oracle.hashgrid_build(p[:, 0], p[:, 1], p[:, 2], cs, (0, 0, 0), dims)
+    counts, offsets, idx = (fh.to_u32(t) for t in grid.query_neighbors_batch(dev(q), 0.03, P))
+    for t in range(0, nq, max(1, nq // 150)):
+        exp = oracle.query_neighbors(q[t], 0.03, p[:, 0], p[:, 1], p[:, 2], cs, (0, 0, 0), dims,
+                                     ocs, osi)
+        assert counts[t] == exp.size
+        assert np.array_equal(idx[offsets[t]:offsets[t + 1]], exp), t
+
+
 @pytest.mark.parametrize("kind", ["subset", "far"])
 def test_query_batch_over_part_of_the_points(fh, gpu_ctx, oracle, kind):
     """A batch that copies the positions reads no more of the caller's arrays than it may: a grid
@@ -151,7 +173,7 @@ def test_query_batch_over_part_of_the_points(fh, gpu_ctx, oracle, kind):
     sub = p[ids]
     ocs, osi, cell = oracle.hashgrid_build(sub[:, 0], sub[:, 1], sub[:, 2], cs, (0, 0, 0), dims)
     near = ids[osi].astype(np.uint32)
-    q = rng.uniform(0.0, 1.0, (2000, 3)).astype(np.float32)
+    q = rng.uniform(0.0, 1.0, (4000, 3)).astype(np.float32)  # enough for the copy
     given = near.copy()
     if kind == "far":
         q[:, 0] *= 0.5  # cells x < 10, rows up to x = 10
