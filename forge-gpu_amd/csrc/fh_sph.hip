@@ -356,6 +356,12 @@ __device__ __forceinline__ Cell3 sph_cell(const float4& p, const GridDesc& g) {
 constexpr int kExactWin = 320;
 // (64 home rows of 3 unions of at most n candidates each: no 32-bit overflow of a stream's length)
 constexpr uint32_t kExactStreamN = 1u << 24;
+// A wave none of whose particles faces more candidates in a slab than this walks them in global memory
+// too: a stream's set-up costs more than it saves, and of the force pass's velocities only the
+// neighbours' are read.  262,000 particles: density pass, 0.3 per cell 24.2 (stream) and 18.8 us, 0.7
+// 25.0 and 22.0, 1 25.5 and 23.4, 2 27.3 and 30.5; force pass, whose registers and LDS leave fewer waves
+// to hide the loads, 0.1 per cell 33.2 and 27.8 us, 0.3 34.8 and 35.7, 1 43.4 and 59.3.
+constexpr uint32_t kExactFewDensity = 16, kExactFewForce = 4;
 struct ExactLds {
     float xyz[3 * (kExactWin + 4)];  // (a row's masked last step reads up to 3 candidates past it)
 };
@@ -403,14 +409,16 @@ template <class Load, class Store, class Row, class One>
 __device__ __forceinline__ void exact_walk(ExactLds& lds, const float4* __restrict__ spos,
                                            uint32_t n, const GridDesc& g,
                                            const uint32_t* __restrict__ cstart, const Cell3& c,
-                                           bool in, int lane, Load&& load, Store&& store,
-                                           Row&& row, One&& one) {
+                                           bool in, int lane, uint32_t few, Load&& load,
+                                           Store&& store, Row&& row, One&& one) {
     const uint32_t hr = (uint32_t)c.cy + (uint32_t)c.cz * g.ny;
     for (int dz = -1; dz <= 1; dz++) {  // uniform
         uint32_t b[3], e[3];
         exact_ranges(c, in, g, cstart, n, dz, b, e);
         LightStream L;
-        bool stream = n <= kExactStreamN && exact_streams(b, e, hr, in, lane);
+        const uint32_t cand = (e[0] - b[0]) + (e[1] - b[1]) + (e[2] - b[2]);
+        bool stream = n <= kExactStreamN && __ballot(cand > few) != 0ull &&
+                      exact_streams(b, e, hr, in, lane);
         if (stream) {
             light_stream(L, b, e, hr, in, lane);
             const uint32_t w = wave_max(L.cnt[0] + L.cnt[1] + L.cnt[2]);
@@ -518,7 +526,7 @@ __global__ __launch_bounds__(kWave) void k_density(const float4* __restrict__ sp
         rho += r2 < h2 ? t : 0.0f;
     };
     exact_walk(
-        lds, spos, n, g, cstart, c, in, lane, [](uint32_t) { return float4{}; },
+        lds, spos, n, g, cstart, c, in, lane, kExactFewDensity, [](uint32_t) { return float4{}; },
         [](int, const float4&) {},
         [&](const float* p, uint32_t, uint32_t m) {
             const float* const pu = p + 3u * (m & ~1u);
@@ -617,7 +625,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8))) v
         }
     };
     exact_walk(
-        lds, spos, n, g, cstart, c, in, lane,
+        lds, spos, n, g, cstart, c, in, lane, kExactFewForce,
         [&](uint32_t j) {
             const float4 v = svel[j];
             return make_float4(v.x, v.y, v.z, srho[j]);
@@ -630,8 +638,11 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8))) v
             });
         },
         [&](uint32_t j) {
-            const float4 q = spos[j], v = svel[j];
-            if (live) pair(q.x, q.y, q.z, v.x, v.y, v.z, srho[j]);
+            const float4 q = spos[j];
+            if (live && exact_r2(pi, q.x, q.y, q.z) < K.h2) {
+                const float4 v = svel[j];
+                pair(q.x, q.y, q.z, v.x, v.y, v.z, srho[j]);
+            }
         });
     if (!in) return;
     if (live) {
@@ -785,7 +796,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8))) v
     };
     const bool live = own && !(rho_i < 1e-6f);
     exact_walk(
-        lds, spos, K.n, g, cstart, sph_cell(pi, g), in, lane,
+        lds, spos, K.n, g, cstart, sph_cell(pi, g), in, lane, kExactFewForce,
         [&](uint32_t j) {
             const float4 v = VISC ? svel[j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             return make_float4(v.x, v.y, v.z, srho[j]);
@@ -798,8 +809,11 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8))) v
             });
         },
         [&](uint32_t j) {
-            const float4 q = spos[j], v = svel[j];
-            if (live) pair(q.x, q.y, q.z, v.x, v.y, v.z, srho[j]);
+            const float4 q = spos[j];
+            if (live && exact_r2(pi, q.x, q.y, q.z) < K.h2) {
+                const float4 v = svel[j];
+                pair(q.x, q.y, q.z, v.x, v.y, v.z, srho[j]);
+            }
         });
     if (live) update(i);
     // a particle that the grid does not hold (rank[s] is then no slot of it)

@@ -162,6 +162,18 @@ def test_step_with_velocities_matches_oracle(fh, gpu_ctx, oracle, mode):
     print("bit-exact fractions", exact)
 
 
+@pytest.mark.parametrize("n", [63, 3000, 20_000, 64_000, 130_000])
+def test_sparse_exact_step_is_bit_exact(fh, gpu_ctx, oracle, n):
+    """0.001 to 2 particles per cell: waves on either side of the few candidates (4 and 16 in a slab)
+    that the bit-exact passes walk in global memory."""
+    from forge_hip import workloads
+    cfg = workloads.small_sph(n=n)
+    rng = np.random.default_rng(n)
+    cfg.x, cfg.y, cfg.z = (rng.uniform(0.0, 1.0, n).astype(np.float32) for _ in range(3))
+    vel = [rng.uniform(-0.5, 0.5, n).astype(np.float32) for _ in range(3)]
+    check_step(fh, oracle, cfg, vel, mode="exact")
+
+
 @pytest.mark.parametrize("per_cell", [5, 8, 10, 11, "mixed"])
 def test_hit_masks_match_oracle(fh, gpu_ctx, oracle, per_cell):
     """Light items with hit masks, one item per wave: rows of 15, 24, 30 and 33 candidates (a mask
