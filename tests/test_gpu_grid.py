@@ -110,9 +110,8 @@ def test_query_batch_matches_oracle(fh, gpu_ctx, oracle):
 @pytest.mark.parametrize("n,nq", [(1, 1), (40, 1025), (3000, 63), (40_000, 1024), (40_000, 1249),
                                   (40_000, 1300)])
 def test_query_batch_sizes_match_oracle(fh, gpu_ctx, oracle, layout, n, nq):
-    """Batches on either side of the copy of the positions (1024 queries, a 32nd of the points),
-    rows shorter and longer than a step of 24 candidates, queries outside the grid; a context too
-    small for the grid's points reads them in place."""
+    """Rows shorter and longer than a step of 16 candidates, queries outside the grid, partial waves; a
+    context too small for the grid's points reads them in place."""
     rng = np.random.default_rng(n + nq)
     cs, dims = 0.05, (20, 20, 20)
     p = rng.uniform(0.0, 1.0, (n, 3)).astype(np.float32)

@@ -43,12 +43,12 @@ def rel_err(a, b):
 
 def set_mode(fh, f, cfg, mode):
     """fast: default work split (below 2^18 particles: items of more than 32 candidates per
-    particle split into 8 parts); fastlarge: the default split of larger systems (192
+    particle split into 8 parts, short ones with hit masks excepted); fastlarge: the default split of larger systems (192
     candidates, 4 parts) at any size; heavy: every (sub-tile, slab) item split into 4
     single-wave parts whose partials are added afterwards; light: none of them (one wavefront per item, shared
     stream); heavy8: as heavy, with 8 parts per item (FH_OPT_HEAVY_PARTS) instead of 4; spill,
     spill8: as heavy and heavy8 with 5 partial-sum slots (FH_OPT_HEAVY_SLOTS), so nearly every
-    item is walked without slots (k_density_pass's part-0 wave, k_force_spill); subcell, subcell2, subcell8: as fast with the cells
+    item is walked without slots (the passes' part-0 waves); subcell, subcell2, subcell8: as fast with the cells
     ordered by 4, 2 or 8 sub-cells per axis (FH_OPT_SUBCELL), so that heavy items skip far
     candidate chunks and compact the others to their near candidates;
     subheavy: every item heavy, with 4 sub-cells per axis; subspill: as subheavy with 5
@@ -174,11 +174,12 @@ def test_sparse_exact_step_is_bit_exact(fh, gpu_ctx, oracle, n):
     check_step(fh, oracle, cfg, vel, mode="exact")
 
 
-@pytest.mark.parametrize("per_cell", [5, 8, 10, 11, "mixed"])
+@pytest.mark.parametrize("per_cell", [5, 6, 8, 10, 11, "mixed"])
 def test_hit_masks_match_oracle(fh, gpu_ctx, oracle, per_cell):
-    """Light items with hit masks, one item per wave: rows of 15, 24, 30 and 33 candidates (a mask
-    word holds 32; an item with a longer row has no masks), streams of one and two windows, and
-    rows of every length beside one another; the bound is the one-step bar of check_step."""
+    """Light items with hit masks: rows of 18, 24 and 30 candidates, streams of one and two windows, and
+    rows of every length beside one another.  Rows of 15 (45 candidates, below the 48 that masks
+    start from) and of 33 (a mask word holds 32) are walked without masks.  The bound is the one-step
+    bar of check_step."""
     from forge_hip import workloads
     cfg = workloads.small_sph(n=4096)
     rng = np.random.default_rng(77)
@@ -192,6 +193,25 @@ def test_hit_masks_match_oracle(fh, gpu_ctx, oracle, per_cell):
     for mode in ("fastlarge", "fast"):  # "fast": short streams whole, the others split
         print(f"hit masks: {per_cell} per cell, {cfg.n} particles, {mode}", flush=True)
         check_step(fh, oracle, cfg, vel, mode=mode)
+
+
+def test_hit_masks_over_kept_streams_match_oracle(fh, gpu_ctx, oracle):
+    """The same from 2^18 particles on, where the plan builds and keeps the candidate streams that both
+    passes walk: 0 to 10 particles per cell, full rows of 30, most items in two windows."""
+    from forge_hip import workloads
+    cfg = workloads.small_sph(n=4096)
+    rng = np.random.default_rng(78)
+    cells = np.array([(x, y, z) for z in range(36) for y in range(40) for x in range(40)])
+    k = rng.integers(0, 11, len(cells))
+    k[(cells[:, 2] > 20) & (cells[:, 0] < 20)] = 10
+    p = (np.repeat(cells, k, axis=0) + rng.uniform(0.02, 0.98, (int(k.sum()), 3))) * cfg.cell_size
+    p = p[rng.permutation(len(p))].astype(np.float32)
+    cfg.n = len(p)
+    assert cfg.n > 1 << 18
+    cfg.x, cfg.y, cfg.z = (np.ascontiguousarray(p[:, a]) for a in range(3))
+    vel = [rng.uniform(-0.5, 0.5, cfg.n).astype(np.float32) for _ in range(3)]
+    print(f"hit masks: {cfg.n} particles", flush=True)
+    check_step(fh, oracle, cfg, vel, mode="fast")
 
 
 def test_c3_step1_matches_oracle(fh, gpu_ctx, oracle):

@@ -69,6 +69,34 @@ def test_density_module_leaves_the_hashgrid(fh, gpu_ctx, oracle, exact):
     assert np.array_equal(u32(f.u32_fields["sorted_indices"]), osi)
 
 
+@pytest.mark.parametrize("dims", [(16, 8, 2), (257, 1, 1), (16, 16, 256), (257, 256, 1),
+                                  (128, 64, 128), (1025, 1024, 1)])
+def test_density_module_grid_with_long_gaps(fh, gpu_ctx, oracle, dims):
+    """Empty cells before, between and behind the runs, with runs at and beside the edges of the
+    256-cell blocks that are filled apart from the slots."""
+    nx, ny, nz = dims
+    C = nx * ny * nz
+    rng = np.random.default_rng(C)
+    edges = np.array([0, 1, 255, 256, 257, 511, 512, 1023, 1024, 1025, 2047, 2048, C // 2, C - 1025,
+                      C - 1024, C - 257, C - 256, C - 2, C - 1])
+    edges = edges[(edges >= 0) & (edges < C)]
+    f = fh.FieldSet(3000)
+    for picks in ([0], [C - 1], [0, C - 1], edges, rng.choice(edges, 4), rng.integers(0, C, 2500)):
+        cells = rng.choice(np.asarray(picks), 3000)
+        cells[:len(picks)] = picks
+        p = [(c + rng.uniform(0.1, 0.9, 3000)).astype(np.float32)
+             for c in (cells % nx, cells // nx % ny, cells // (nx * ny))]
+        for nm, a in zip(("pos_x", "pos_y", "pos_z"), p):
+            f.f32_fields[nm] = dev(a)
+        f.context(C)
+        torch.cuda.synchronize()
+        fh.SphDensityModule(1.0, 1.0, dims, 1.0).execute(f, 1e-4)
+        f.context().sync()
+        ocs, osi, _ = oracle.hashgrid_build(*p, 1.0, (0, 0, 0), dims)
+        assert np.array_equal(u32(f.u32_fields["cell_start"]), ocs)
+        assert np.array_equal(u32(f.u32_fields["sorted_indices"]), osi)
+
+
 @pytest.mark.parametrize("which", ["pressure", "viscosity"])
 @pytest.mark.parametrize("case", ["c0", "clumps"])
 def test_unfused_pass_is_bit_exact(fh, gpu_ctx, oracle, which, case):
@@ -132,8 +160,8 @@ def test_unfused_pipeline_is_bit_exact(fh, gpu_ctx, oracle):
 
 def shuffled_grid(kind, cfg, oracle, rng):
     """A grid the exact walks must not take for one of these positions, or that they walk in its
-    edge cases: positions moved since the build, particles missing from it or held twice, ids
-    beyond n, a sparse row beside a dense one (streams far longer than the lanes' ranges)."""
+    edge cases: positions moved since the build, or a sparse row beside a dense one (streams far
+    longer than the lanes' ranges)."""
     if kind == "sparse":
         k = cfg.n // 2
         cfg.x[:k] = rng.uniform(0.0, 1.0, k)
@@ -177,9 +205,9 @@ def test_unfused_pass_over_other_grids_is_bit_exact(fh, gpu_ctx, oracle, which, 
 
 @pytest.mark.parametrize("which", ["pressure", "viscosity"])
 def test_unfused_pass_over_a_malformed_grid(fh, gpu_ctx, oracle, which):
-    """Ids beyond n are no neighbours; a particle the grid holds twice is updated once, one that it
-    does not hold (its slot is taken by the duplicate) from its own position: what the CPU
-    restatement computes with the bad slots removed from the neighbour lists."""
+    """Ids beyond n are no neighbours, and a particle that the grid does not hold (its slot holds such
+    an id) is walked from its own position: what the CPU restatement computes with the bad slots
+    removed from the neighbour lists."""
     from forge_hip import workloads
     cfg = workloads.small_sph(n=5000, cols=16)
     vel = state(cfg, 5)
@@ -211,3 +239,38 @@ def test_unfused_pass_over_a_malformed_grid(fh, gpu_ctx, oracle, which):
         got = f.f32_fields[nm].cpu().numpy()
         assert np.array_equal(got, ref[c][:cfg.n]), nm
     assert not np.array_equal(ref[0][gone], vel[0][gone])  # the missing ones moved as well
+
+
+@pytest.mark.parametrize("which", ["pressure", "viscosity"])
+@pytest.mark.parametrize("shift", [1, 7, 2500])
+def test_unfused_pass_over_a_grid_with_duplicates(fh, gpu_ctx, oracle, which, shift):
+    """A particle that the grid holds twice (beside its own slot, in its neighbourhood or in a far
+    cell) is a neighbour twice and is updated once; one whose slot the duplicate takes is walked
+    from its own position: bit for bit the CPU restatement over the same lists."""
+    from forge_hip import workloads
+    cfg = workloads.small_sph(n=5000, cols=16)
+    vel = state(cfg, 6)
+    ocs, osi, _ = oracle.hashgrid_build(cfg.x, cfg.y, cfg.z, cfg.cell_size, (0, 0, 0), cfg.dims)
+    prm = oracle.sph_params(cfg.h, cfg.cell_size, cfg.dims, cfg.mass, cfg.gas_constant,
+                            cfg.rest_density, cfg.viscosity)
+    rho = oracle.sph_density(prm, cfg.x, cfg.y, cfg.z, ocs, osi)
+    ids = osi.copy()
+    at = np.arange(50, cfg.n - shift, 97)
+    ids[at] = osi[at + shift]
+    twice, gone = osi[at + shift], osi[at]
+    assert np.bincount(ids, minlength=cfg.n)[twice].min() >= 2
+    ref = (oracle.sph_pressure if which == "pressure" else oracle.sph_viscosity)(
+        prm, cfg.x, cfg.y, cfg.z, *vel, rho, ocs, ids, cfg.dt)
+    f = fieldset(fh, cfg, vel)
+    f.f32_fields["density"] = dev(rho)
+    f.u32_fields["cell_start"] = fh.from_u32(ocs)
+    f.u32_fields["sorted_indices"] = fh.from_u32(ids)
+    _, p, v = modules(fh, cfg)
+    f.context(cfg.num_cells)
+    torch.cuda.synchronize()
+    (p if which == "pressure" else v).execute(f, cfg.dt)
+    f.context().sync()
+    for c, nm in enumerate(("vel_x", "vel_y", "vel_z")):
+        assert np.array_equal(f.f32_fields[nm].cpu().numpy(), ref[c]), nm
+    for some in (twice, gone):
+        assert not np.array_equal(ref[0][some], vel[0][some])
