@@ -220,7 +220,7 @@ struct fh_ctx {
     float* fpart;        // [3][3][max_n] per-slab acceleration partials (fast kernels)
     uint32_t* heavy;     // [kHeavyLists][heavy_cap] heavy (64-particle tile, slab) work items
     uint32_t heavy_cap;  // entries per heavy sub-list
-    uint8_t* heavy_flag; // [3 * ceil(max_n / 64)] 1: heavy list, 2: co-located, skipped
+    uint8_t* heavy_flag; // [3 * ceil(max_n / 64)] item flags: light, heavy list, light with hit masks
     float* hpart;        // heavy work partials: per slot, hpart_parts x 4 x 64 floats
     uint32_t hpart_parts; // parts per slot the buffer has room for (kHeavyWaves until 8 are asked for)
     uint32_t hslot_cap;  // partial-sum slots in hpart (FH_OPT_HEAVY_SLOTS; default: every item)
@@ -458,7 +458,7 @@ hipError_t launch_prep(fh_ctx* c, const SphArgs& a);
 // work plan of the fast passes.
 hipError_t launch_group_plan(fh_ctx* c, const SphArgs& a, bool with_vel);
 // New state in sorted order (c->sout); with `to_particles`, also moved to the caller's arrays
-// (`rebuild_rank`: first recompute c->rank from the particle ids, after resident substeps).
+// (`rebuild_rank`: c->rank from the particle ids first, after resident substeps; with forces).
 // `next_keys` (may be null) receives the cell of each new position, the keys of the next
 // resident substep.
 hipError_t launch_finalize(fh_ctx* c, const SphArgs& a, const fh_epilogue* epi,

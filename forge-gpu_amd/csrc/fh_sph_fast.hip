@@ -1612,7 +1612,10 @@ __device__ __forceinline__ void force_trans(const float4* __restrict__ rec,
 // Acceleration partials: fpart[slab][c][s] = sum over the slab's neighbours j of the pressure
 // and viscosity pair terms (sph_fused.rs:604-623), not yet divided by rho_i.  Same windowed
 // stream as density_light; the window is staged by copying force records (k_prep).
-// MASKED: the hits of the density pass's masks only.
+// MASKED: the hits of the density pass's masks only.  A mask bit is the sign of h^2 - r^2 as the
+// density pass rounds it, force_pair's own test that of r^2 + 1e-30 < h^2: a pair within a rounding of h
+// may pass the second with its bit clear, so that the sums are those of the full walk but for terms
+// whose h - r is of rounding size.
 template <bool MASKED>
 __device__ __forceinline__ void force_light(uint32_t item, int lane, float4* bp, float4* bv,
                                             const float4* __restrict__ spos,
@@ -1996,8 +1999,7 @@ __global__ __launch_bounds__(256) void k_finalize(const float4* __restrict__ spo
     o[0] = make_float4(npx, npy, npz, rho);
     o[1] = make_float4(nvx, nvy, nvz, v.w);  // .w: the particle id
     if (keys_out) keys_out[s] = sort_key_of(npx, npy, npz, g);  // the next resident substep's keys
-    // the last of several resident substeps: the particle -> slot map for k_scatter (what
-    // k_rank_of would read back from the new state)
+    // the last of several resident substeps: the particle -> slot map for k_scatter
     if (rank_out && __float_as_uint(v.w) < n) rank_out[__float_as_uint(v.w)] = s;
     if (want_accel) o[2] = make_float4(ax, ay, az, 0.0f);
 }
@@ -2146,16 +2148,6 @@ hipError_t launch_force_fast(fh_ctx* c, const SphArgs& a, const uint32_t* cell_s
     return e;
 }
 
-// rank[id] = s for the particle id carried in the new state of slot s (sout[2 s + 1].w): the
-// particle -> slot map after resident substeps.
-__global__ __launch_bounds__(256) void k_rank_of(const float4* __restrict__ sout, uint32_t n,
-                                                 uint32_t* __restrict__ rank) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const uint32_t i = __float_as_uint(sout[2u * s + 1u].w);
-    if (i < n) rank[i] = s;
-}
-
 hipError_t launch_finalize(fh_ctx* c, const SphArgs& a, const fh_epilogue* epi, bool density_only,
                            float* px, float* py, float* pz, float* vx, float* vy, float* vz,
                            float* density, float* accel, bool to_particles, bool rebuild_rank,
@@ -2174,21 +2166,14 @@ hipError_t launch_finalize(fh_ctx* c, const SphArgs& a, const fh_epilogue* epi, 
     }
     F.e = epi ? epi->restitution : 0.0f;
     tbeg(c, KID_FINAL);
-    // after resident substeps k_finalize itself writes the particle -> slot map (with forces: a
-    // density-only call returns before it has the particle id)
-    const bool rank_here = to_particles && rebuild_rank && !density_only;
     const auto fin = heavy_parts(c, a.n) == 8u ? k_finalize<8> : k_finalize<kHeavyWaves>;
     fin<<<ceil_div(a.n, 256u), 256, 0, c->stream>>>(c->spos, c->svel, c->dpart, c->fpart,
                                                            c->wpart, a.n, c->max_n, F,
                                                            accel != nullptr, c->sout, a.g,
                                                            density_only ? nullptr : next_keys,
                                                            c->hslot, c->hpart, c->srho,
-                                                           rank_here ? c->rank : nullptr);
+                                                           to_particles && rebuild_rank ? c->rank : nullptr);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && to_particles && rebuild_rank && !rank_here) {
-        k_rank_of<<<ceil_div(a.n, 256u), 256, 0, c->stream>>>(c->sout, a.n, c->rank);
-        e = hipGetLastError();
-    }
     if (e == hipSuccess && to_particles) {
         k_scatter<<<ceil_div(a.n, 256u), 256, 0, c->stream>>>(c->sout, c->rank, a.n, F.flags,
                                                               px, py, pz, vx, vy, vz, density,
