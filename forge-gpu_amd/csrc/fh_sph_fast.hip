@@ -845,8 +845,8 @@ static_assert(kLightCacheWords == kLightHead + kWin, "light stream cache layout"
 
 // Light items stage a window as x, y, z, 12 bytes per candidate.  Their rows are bound by the LDS,
 // and lanes of different cells read about a cell's worth of candidates apart: at 16 bytes a fluid
-// of eight particles per cell puts those reads 128 bytes apart, on the same banks (16.8 LDS cycles
-// per candidate, 8.8 of them conflicts).  1,048,576 particles of a dam-break block: density pass
+// of eight particles per cell puts those reads 128 bytes apart, on the same banks (8.7 conflict cycles
+// per LDS instruction, 0.7 with 12 bytes).  1,048,576 particles of a dam-break block: density pass
 // 115 -> 61 us (69 with the hit masks below); a sparse state is unchanged.
 constexpr int kPad = 4;  // candidates of readable LDS behind a window
 
