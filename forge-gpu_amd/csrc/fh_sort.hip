@@ -241,7 +241,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hash_hist(
 // Sum the partial rows: workgroup (r, b) adds rows r*R .. r*R+R-1 of histogram slots
 // 256 b .. 256 b + 255 into the histograms.  (No fence / last-workgroup election here: an
 // agent-scope release on this part writes the L2 back, which costs tens of microseconds per
-// workgroup; the decision about the passes is a separate one-workgroup kernel, the kernel
+// workgroup; the passes' workgroups decide from the marks left here, sort_plan, and the kernel
 // boundary gives the visibility.)
 // First-pass prefixes (pre != null: a small sort, whose histogram rows are its 4096-key chunks,
 // rpt of them per first-pass tile): for the first pass's digits (slots < nb0), this workgroup's
