@@ -294,42 +294,103 @@ __global__ __launch_bounds__(kWave) void k_nbr_stream(const float4* __restrict__
 // neighbours each (2.6 candidates per point) 106 us against 145 in place; 2 (1.3) 114 against 104; 0.5
 // (0.3) 95 against 64.  600,000 points, 30 neighbours: 7,000 queries (2.3) 38 against 34.  100,000
 // points and queries: 3 neighbours (19) 30 against 33, 1 (6.4) 28 against 24.  Below kQueryCopyMin
-// queries the extra launch would cost more than it gives.  The points' number is the grid's own
-// (cell_start[C]), read on the device; a grid of more points than the context holds is read in place.
+// queries the extra launch would cost more than it gives.  Queries all over the grid meet 27 n / C
+// candidates each, wherever the points are.  Where that is too few, but the queries are at least a
+// kQueryFew-th of the points, they may all be where the points are (a fluid in a corner of its box):
+// k_sort_pos counts the candidates of kQuerySamples of them and leaves its answer for k_query (5 us:
+// 120,000 queries among 600,000 points in a 64th of the grid 72 us a pass, 263 in place).
+// The points' number is the grid's own (cell_start[C]), read on the device; a grid of more points than
+// the context holds is read in place.
 // An id of that number or more (a grid over some of an array's points, an entry that no query comes
 // near) is not followed by the copy, which leaves a NaN: its position is read where a query meets it.
 constexpr uint32_t kQueryLanes = 8, kQueryStep = 2, kQueryCopyMin = 1024;
 constexpr uint32_t kQueryCopyShare = 5, kQueryCacheShare = 24, kQueryCacheN = 1u << 18;
+constexpr uint32_t kQueryFew = 32, kQuerySamples = 16;
 struct QueryCopy {
     Pos3* spos;      // null: no copy (12 bytes: a row is a quarter fewer lines than with float4)
-    uint32_t max_n;  // its room
+    uint32_t* ask;   // k_sort_pos' answer where query_rule asks for the samples
+    uint32_t max_n;  // room of spos
     uint32_t nq;     // queries of the whole batch
     uint32_t C;      // cells
 };
-// Whether the batch meets at least `share` / 2 candidates per point of the grid: 27 n / C per query.
-__host__ __device__ __forceinline__ bool query_candidates(uint32_t nq, uint32_t C, uint32_t share) {
-    return (uint64_t)nq * 54u >= (uint64_t)C * share;
-}
-__host__ __device__ __forceinline__ uint32_t query_share(uint32_t n) {
+__device__ __forceinline__ uint32_t query_share(uint32_t n) {
     return n < kQueryCacheN ? kQueryCacheShare : kQueryCopyShare;
 }
-__device__ __forceinline__ bool query_copied(const QueryCopy& Q, uint32_t n) {
-    return Q.spos && n <= Q.max_n && query_candidates(Q.nq, Q.C, query_share(n));
+// Whether the batch reads from a copy: by kQueryCopyShare / 2 candidates per point of the grid.
+enum : uint32_t { kInPlace, kCopied, kAsk };
+__device__ __forceinline__ uint32_t query_rule(const QueryCopy& Q, uint32_t n) {
+    if (!Q.spos || n > Q.max_n) return kInPlace;
+    if ((uint64_t)Q.nq * 54u >= (uint64_t)Q.C * query_share(n)) return kCopied;
+    return (uint64_t)Q.nq * kQueryFew >= n ? kAsk : kInPlace;
+}
+
+// The cell of a query (not clamped) and its row r = (dz + 1) * 3 + dy + 1 of the reference's walk.
+struct QueryCell {
+    int64_t cy, cz, x0, x1;
+};
+__device__ __forceinline__ QueryCell query_cell(float px, float py, float pz, const GridDesc& g) {
+    const int64_t cx = rust_as_i32(floorf((px - g.ox) / g.cs));
+    QueryCell c;
+    c.cy = rust_as_i32(floorf((py - g.oy) / g.cs));
+    c.cz = rust_as_i32(floorf((pz - g.oz) / g.cs));
+    c.x0 = cx - 1 < 0 ? 0 : cx - 1;
+    c.x1 = cx + 1 > (int64_t)g.nx - 1 ? (int64_t)g.nx - 1 : cx + 1;
+    return c;
+}
+__device__ __forceinline__ void query_range(const QueryCell& c, uint32_t r, const GridDesc& g,
+                                            const uint32_t* __restrict__ cstart, uint32_t n,
+                                            uint32_t& b, uint32_t& e) {
+    const int64_t nz = c.cz + (int64_t)(r / 3u) - 1, ny = c.cy + (int64_t)(r % 3u) - 1;
+    b = e = 0u;
+    if (nz < 0 || nz >= (int64_t)g.nz || ny < 0 || ny >= (int64_t)g.ny || c.x0 > c.x1) return;
+    const uint32_t row = (uint32_t)ny * g.nx + (uint32_t)nz * g.nx * g.ny;
+    e = min(cstart[row + (uint32_t)c.x1 + 1u], n);
+    b = cstart[row + (uint32_t)c.x0];
 }
 
 __global__ __launch_bounds__(256) void k_sort_pos(const float* __restrict__ x,
                                                   const float* __restrict__ y,
                                                   const float* __restrict__ z, uint32_t stride,
+                                                  GridDesc g,
                                                   const uint32_t* __restrict__ cstart,
                                                   const uint32_t* __restrict__ sidx,
+                                                  const float* __restrict__ qx,
+                                                  const float* __restrict__ qy,
+                                                  const float* __restrict__ qz, uint32_t qstride,
                                                   QueryCopy Q) {
     const uint32_t n = cstart[Q.C];
-    if (!query_copied(Q, n)) return;
+    const uint32_t rule = query_rule(Q, n);
+    if (rule == kInPlace) return;
+    if (rule == kAsk) {  // the same count in every workgroup
+        __shared__ uint32_t s_met;
+        if (threadIdx.x < kWave) {
+            uint32_t met = 0;
+            if (threadIdx.x < kQuerySamples) {
+                const size_t o = (size_t)((uint64_t)threadIdx.x * Q.nq / kQuerySamples) * qstride;
+                const QueryCell c = query_cell(qx[o], qy[o], qz[o], g);
+#pragma unroll
+                for (uint32_t r = 0; r < 9u; r++) {
+                    uint32_t b, e;
+                    query_range(c, r, g, cstart, n, b, e);
+                    met += e > b ? min(e - b, 1u << 22) : 0u;  // (no overflow: 144 rows)
+                }
+            }
+#pragma unroll
+            for (int d = 1; d < (int)kQuerySamples; d <<= 1)
+                met += (uint32_t)__shfl_xor((int)met, d, kWave);
+            if (threadIdx.x == 0u) s_met = met;
+        }
+        __syncthreads();
+        const bool copy =
+            2u * (uint64_t)s_met * Q.nq >= (uint64_t)kQuerySamples * query_share(n) * n;
+        if (blockIdx.x == 0u && threadIdx.x == 0u) *Q.ask = copy ? 1u : 0u;
+        if (!copy) return;
+    }
     for (uint32_t s = blockIdx.x * 256u + threadIdx.x; s < n; s += gridDim.x * 256u) {
         const uint32_t i = sidx[s];
-        const size_t o = (size_t)(i < n ? i : 0u) * stride;
+        const size_t at = (size_t)(i < n ? i : 0u) * stride;
         const float nan = __builtin_nanf("");
-        Pos3 p = {x[o], y[o], z[o]};
+        Pos3 p = {x[at], y[at], z[at]};
         if (i >= n) p = Pos3{nan, nan, nan};
         Q.spos[s] = p;
     }
@@ -352,27 +413,15 @@ __global__ __launch_bounds__(256) void k_query(const float* __restrict__ x,
     const uint32_t qi = (blockIdx.x * 256u + threadIdx.x) / kQueryLanes;
     if (qi >= nq) return;  // whole groups
     const uint32_t n = cstart[Q.C];
-    const bool copied = query_copied(Q, n);  // uniform
+    const uint32_t rule = query_rule(Q, n), asked = *Q.ask;
+    const bool copied = rule == kCopied || (rule == kAsk && asked);  // uniform
     const size_t oq = (size_t)qi * qstride;
     const float px = qx[oq], py = qy[oq], pz = qz[oq];
-    const int64_t cx = rust_as_i32(floorf((px - g.ox) / g.cs));
-    const int64_t cy = rust_as_i32(floorf((py - g.oy) / g.cs));
-    const int64_t cz = rust_as_i32(floorf((pz - g.oz) / g.cs));
-    const int64_t x0 = cx - 1 < 0 ? 0 : cx - 1;
-    const int64_t x1 = cx + 1 > (int64_t)g.nx - 1 ? (int64_t)g.nx - 1 : cx + 1;
-    // row r = (dz + 1) * 3 + dy + 1 of the reference's walk: lane t loads row t's range, lane 0
-    // also the last one's
-    const auto range = [&](uint32_t r, uint32_t& b, uint32_t& e) {
-        const int64_t nz = cz + (int64_t)(r / 3u) - 1, ny = cy + (int64_t)(r % 3u) - 1;
-        b = e = 0u;
-        if (nz < 0 || nz >= (int64_t)g.nz || ny < 0 || ny >= (int64_t)g.ny || x0 > x1) return;
-        const uint32_t row = (uint32_t)ny * g.nx + (uint32_t)nz * g.nx * g.ny;
-        e = min(cstart[row + (uint32_t)x1 + 1u], n);
-        b = cstart[row + (uint32_t)x0];
-    };
+    const QueryCell c = query_cell(px, py, pz, g);
+    // lane t loads row t's range, and every lane the last one's
     uint32_t b0, e0, b8, e8;
-    range(t, b0, e0);
-    range(8u, b8, e8);
+    query_range(c, t, g, cstart, n, b0, e0);
+    query_range(c, 8u, g, cstart, n, b8, e8);
     uint32_t cnt = 0;
     uint32_t* out = (offsets && indices) ? indices + offsets[qi] : nullptr;
     const uint32_t room = out ? offsets[qi + 1] - offsets[qi] : 0u;
@@ -439,13 +488,12 @@ hipError_t launch_query(fh_ctx* c, const float* x, const float* y, const float* 
                         const float* qz, uint32_t qstride, uint32_t nq, float radius,
                         uint32_t* counts, const uint32_t* offsets, uint32_t* indices) {
     if (nq == 0) return hipSuccess;
-    const uint32_t C = g.nx * g.ny * g.nz;
-    const bool copy = nq >= kQueryCopyMin && query_candidates(nq, C, query_share(c->max_n));
-    const QueryCopy Q{copy ? (Pos3*)c->spos : nullptr, c->max_n, nq, C};
+    const QueryCopy Q{nq >= kQueryCopyMin ? (Pos3*)c->spos : nullptr, &c->ctl->query_copy, c->max_n,
+                      nq, g.nx * g.ny * g.nz};
     if (Q.spos) {
         const uint32_t groups = ceil_div(c->max_n, 256u);
         k_sort_pos<<<groups < 2048u ? groups : 2048u, 256, 0, c->stream>>>(
-            x, y, z, stride, cell_start, sorted_indices, Q);
+            x, y, z, stride, g, cell_start, sorted_indices, qx, qy, qz, qstride, Q);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

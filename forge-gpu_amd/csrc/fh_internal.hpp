@@ -132,7 +132,7 @@ struct Control {
     uint32_t epoch;                     // bumped by k_begin before each sort / scan
     uint32_t plan;                      // bit p: sort pass p runs (written by pass 0)
     uint32_t spin_limit;                // look-back polls before giving up (0: kSpinLimit)
-    uint32_t pad0;
+    uint32_t query_copy;                // k_sort_pos' answer for k_query (QueryCopy::ask)
     uint32_t* host_error;               // pinned host word of a context that a failure is stored to,
                                         // or null: to `error` (the no-alloc sort)
     uint32_t pad1[26];

@@ -160,6 +160,33 @@ def test_query_batch_rules_match_oracle(fh, gpu_ctx, oracle, n, nq):
         assert np.array_equal(idx[offsets[t]:offsets[t + 1]], exp), t
 
 
+@pytest.mark.parametrize("where", ["points", "elsewhere", "all over"])
+@pytest.mark.parametrize("nq", [1249, 1250, 3000])
+def test_query_batch_of_points_in_a_corner(fh, gpu_ctx, oracle, where, nq):
+    """40,000 points in a corner of the grid: batches of a 32nd of the points on count the candidates of
+    a few of their queries, which are many, none, or some, to decide for the copy; a second batch on
+    the same context decides anew."""
+    rng = np.random.default_rng(nq)
+    cs, dims, n = 0.05, (20, 20, 20), 40_000
+    p = rng.uniform(0.0, 0.25, (n, 3)).astype(np.float32)
+    q = rng.uniform(0.0, 1.0, (nq, 3))
+    q = (q if where == "all over" else 0.25 * q + (0.0 if where == "points" else 0.6))
+    q = q.astype(np.float32)
+    grid = fh.HashGrid(cs, dims, (0, 0, 0), n, ctx=gpu_ctx)
+    P = dev(p)
+    grid.build(P)
+    ocs, osi, _ = oracle.hashgrid_build(p[:, 0], p[:, 1], p[:, 2], cs, (0, 0, 0), dims)
+    for batch in (q, q[::-1].copy()):
+        got = grid.query_neighbors_batch(dev(batch), 0.01, P)
+        counts, offsets, idx = (fh.to_u32(t) for t in got)
+        for t in range(0, nq, max(1, nq // 100)):
+            exp = oracle.query_neighbors(batch[t], 0.01, p[:, 0], p[:, 1], p[:, 2], cs, (0, 0, 0),
+                                         dims, ocs, osi)
+            assert counts[t] == exp.size
+            assert np.array_equal(idx[offsets[t]:offsets[t + 1]], exp), t
+        grid.query_neighbors_batch(dev(batch + 0.3), 0.01, P)
+
+
 @pytest.mark.parametrize("kind", ["subset", "far"])
 def test_query_batch_over_part_of_the_points(fh, gpu_ctx, oracle, kind):
     """A batch that copies the positions reads no more of the caller's arrays than it may: a grid
